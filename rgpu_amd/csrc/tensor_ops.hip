@@ -9,10 +9,11 @@
 //   broadcast binary ops          tensor.rs:183-246
 //   reduce_to                     tensor.rs:399-438 (per output element, source order: exact)
 //   sum / mean of all elements    tensor.rs:279-286 (fixed-order two-stage tree)
-//   softmax_rows and its VJP      tensor.rs:455-472, ops.rs:291-309 (one thread per row, sequential)
+//   softmax_rows and its VJP      tensor.rs:455-472, ops.rs:291-309 (row sums in column order: exact)
 //   mae / softmax-xent / bce      losses.rs:46-53, 99-115, 143-162
 
 #include <algorithm>
+#include <type_traits>
 
 #include "rt_internal.h"
 
@@ -187,11 +188,21 @@ __global__ __launch_bounds__(256) void sum_stage1(const float* __restrict__ x, l
   }
 }
 
-__global__ void sum_stage2(const float* __restrict__ part, int parts, float div, float* __restrict__ out) {
-  if (threadIdx.x != 0 || blockIdx.x != 0) return;
+// out[0] = (the parts added) / div: thread t adds parts t, t + 256, ... in
+// order, then a shared-memory tree.  One thread walking the parts alone was a
+// chain of dependent loads (512 parts: SUM1_US us; SUM2_US us this way).
+__global__ __launch_bounds__(256) void sum_stage2(const float* __restrict__ part, int parts, float div,
+                                                  float* __restrict__ out) {
+  __shared__ float sh[256];
   float acc = 0.0f;
-  for (int i = 0; i < parts; ++i) acc += part[i];
-  out[0] = acc / div;
+  for (int i = threadIdx.x; i < parts; i += 256) acc += part[i];
+  sh[threadIdx.x] = acc;
+  __syncthreads();
+  for (int w = 128; w > 0; w >>= 1) {
+    if ((int)threadIdx.x < w) sh[threadIdx.x] += sh[threadIdx.x + w];
+    __syncthreads();
+  }
+  if (threadIdx.x == 0) out[0] = sh[0] / div;
 }
 
 // out[i] = (s[0] / div) * (x ? x[i] : 1): the VJPs of sum / mean (Tensor::full)
@@ -204,34 +215,206 @@ __global__ __launch_bounds__(256) void scalar_fill_kernel(const float* __restric
     out[i] = x ? x[i] * v : v;
 }
 
-// tensor.rs:455-472: max, exp and a sequential sum, then divide; one thread per row.
-__global__ __launch_bounds__(256) void softmax_rows_kernel(const float* __restrict__ z, float* __restrict__ y,
-                                                           long long rows, long long cols) {
-  const long long i = blockIdx.x * 256LL + threadIdx.x;
-  if (i >= rows) return;
-  const float* row = z + i * cols;
-  float* dst = y + i * cols;
-  float mx = -INFINITY;
-  for (long long j = 0; j < cols; ++j) mx = fmaxf(mx, row[j]);
-  float sum = 0.0f;
-  for (long long j = 0; j < cols; ++j) {
-    const float e = expf(row[j] - mx);
-    dst[j] = e;
-    sum += e;
+// Row kernels (softmax, its VJP, softmax cross-entropy from the logits).  A
+// block takes a band of G·NR rows, G = T / L groups of L lanes with NR rows
+// each, a lane holding columns l, l + L, ... of its rows in R registers: rows
+// are read once, in whole cache lines, and written once.  The sums over a
+// row (Σ exp, Σ g·s) keep the reference's left-to-right order, hence its
+// bits: the terms go to LDS and one lane per row adds that row, all rows of
+// the band side by side, about 2 us per 1000 columns.  What bounds them is
+// HBM, then that chain.  One thread per row, each walking its row in memory
+// alone, read a cache line per lane and step: 4096 x 1000 softmax and VJP
+// 864 + 901 us, SM_NEW_US us this way.
+typedef float f4t __attribute__((ext_vector_type(4)));
+
+template <int L_, int R_, int NR_, int T_>
+struct Band {
+  static constexpr int L = L_, R = R_, NR = NR_, T = T_, G = T / L, ROWS = G * NR;
+  // Row pitch in LDS (floats): 16-byte rows an odd number of 16 bytes apart,
+  // so the adding lanes' b128 reads fall into different banks.
+  static constexpr int PITCH = (L * R / 8) * 8 + 4;
+  static constexpr int SMEM = ROWS * PITCH;
+  static_assert(ROWS <= T, "one adding lane per row");
+
+  float v[NR][R];
+
+  // This lane's columns of the band's rows from row0, all loads issued
+  // together.  Past the last row or column they repeat it (rows, cols >= 1).
+  __device__ inline void load(const float* m, long long row0, long long rows, int cols) {
+    const int lane = threadIdx.x % L;
+#pragma unroll
+    for (int n = 0; n < NR; ++n) {
+      const float* row = m + min(row0 + group_row(n), rows - 1) * cols;
+#pragma unroll
+      for (int q = 0; q < R; ++q) v[n][q] = row[min(lane + L * q, cols - 1)];
+    }
   }
-  for (long long j = 0; j < cols; ++j) dst[j] = dst[j] / sum;
+  __device__ static inline int group_row(int n) { return threadIdx.x / L + G * n; }
+  // f(n, q, column) for this lane's columns.
+  template <class F>
+  __device__ static inline void each(int cols, F&& f) {
+    const int lane = threadIdx.x % L;
+#pragma unroll
+    for (int n = 0; n < NR; ++n)
+#pragma unroll
+      for (int q = 0; q < R; ++q)
+        if (lane + L * q < cols) f(n, q, lane + L * q);
+  }
+  // v = exp(v - row max).
+  __device__ inline void exponentials(int cols) {
+    const int lane = threadIdx.x % L;
+#pragma unroll
+    for (int n = 0; n < NR; ++n) {
+      float mx = -INFINITY;
+#pragma unroll
+      for (int q = 0; q < R; ++q)
+        if (lane + L * q < cols) mx = fmaxf(mx, v[n][q]);
+#pragma unroll
+      for (int off = L / 2; off > 0; off >>= 1) mx = fmaxf(mx, __shfl_xor(mx, off, 64));
+#pragma unroll
+      for (int q = 0; q < R; ++q)
+        if (lane + L * q < cols) v[n][q] = expf(v[n][q] - mx);
+    }
+  }
+  // sums[r] = the terms of row r added in column order; put(n, q) is the term.
+  template <class F>
+  __device__ inline void add_rows(int cols, float* sh, float* sums, F&& put) const;
+};
+
+// acc + p[0] + p[1] + ... + p[n - 1], one add after another; p is 16-byte
+// aligned.  Two batches of 32 terms take turns: one is on its way from LDS
+// while the other is added, so the chain waits on its own adds only.
+__device__ inline float add_in_order(float acc, const float* p, int n) {
+  const f4t* q = reinterpret_cast<const f4t*>(p);
+  auto fetch = [&](f4t (&t)[8], int j) {
+#pragma unroll
+    for (int u = 0; u < 8; ++u) t[u] = q[j / 4 + u];
+  };
+  auto add = [&](const f4t (&t)[8]) {
+#pragma unroll
+    for (int u = 0; u < 8; ++u)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) acc += t[u][e];
+  };
+  const int whole = n & ~31;
+  if (whole > 0) {
+    // Fetches past the end repeat the last batch: a branch there would make
+    // the compiler wait for both batches.
+    f4t a[8], b[8];
+    fetch(a, 0);
+    int j = 0;
+    for (; j + 64 <= whole; j += 64) {
+      fetch(b, j + 32);
+      add(a);
+      fetch(a, min(j + 64, whole - 32));
+      add(b);
+    }
+    if (j < whole) add(a);
+  }
+  for (int j = whole; j < n; ++j) acc += p[j];
+  return acc;
 }
 
-// ops.rs:291-309: dx = s ⊙ (g − Σ_j g_j s_j), per row, sequential dot.
-__global__ __launch_bounds__(256) void softmax_rows_vjp_kernel(const float* __restrict__ s, const float* __restrict__ g,
-                                                               float* __restrict__ dx, long long rows, long long cols) {
-  const long long i = blockIdx.x * 256LL + threadIdx.x;
-  if (i >= rows) return;
-  const float* sr = s + i * cols;
-  const float* gr = g + i * cols;
-  float dot = 0.0f;
-  for (long long j = 0; j < cols; ++j) dot += gr[j] * sr[j];
-  for (long long j = 0; j < cols; ++j) dx[i * cols + j] = sr[j] * (gr[j] - dot);
+template <int L_, int R_, int NR_, int T_>
+template <class F>
+__device__ inline void Band<L_, R_, NR_, T_>::add_rows(int cols, float* sh, float* sums, F&& put) const {
+  each(cols, [&](int n, int q, int col) { sh[group_row(n) * PITCH + col] = put(n, q); });
+  __syncthreads();
+  if (threadIdx.x < ROWS) sums[threadIdx.x] = add_in_order(0.0f, sh + threadIdx.x * PITCH, cols);
+  __syncthreads();
+}
+
+// The row kernels for rows too long for a lane group's registers: a block of
+// four waves takes four rows, one per wave, in chunks of kLongChunk columns
+// through LDS; z (or s and g) is read again for the results.
+constexpr int kRowThreads = 256, kLossThreads = 1024, kLongChunk = 2048;
+constexpr int kLongPitch = kLongChunk + 4, kLongRows = kRowThreads / 64;
+
+__device__ inline float wave_max_row(const float* row, long long cols) {
+  float mx = -INFINITY;
+  for (long long j = threadIdx.x & 63; j < cols; j += 64) mx = fmaxf(mx, row[j]);
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) mx = fmaxf(mx, __shfl_xor(mx, off, 64));
+  return mx;
+}
+
+// The in-order sum of term(j), j < cols, of this wave's row.  Every thread of
+// the block takes part; `in`: the wave has a row.
+template <class F>
+__device__ inline float long_row_sum(long long cols, bool in, float* sh, F&& term) {
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  __shared__ float sums[kLongRows];
+  float acc = 0.0f;
+  for (long long c0 = 0; c0 < cols; c0 += kLongChunk) {
+    const int n = (int)min((long long)kLongChunk, cols - c0);
+    if (in)
+      for (int j = lane; j < n; j += 64) sh[wave * kLongPitch + j] = term(c0 + j);
+    __syncthreads();
+    if (threadIdx.x < kLongRows) acc = add_in_order(acc, sh + threadIdx.x * kLongPitch, n);
+    __syncthreads();
+  }
+  if (threadIdx.x < kLongRows) sums[threadIdx.x] = acc;
+  __syncthreads();
+  const float v = sums[wave];
+  __syncthreads();
+  return v;
+}
+
+// tensor.rs:455-472: max, exp, sum, then divide.  y may be z.
+template <class B>
+__global__ __launch_bounds__(B::T) void softmax_rows_kernel(const float* z, float* y, long long rows, int cols) {
+  __shared__ __attribute__((aligned(16))) float sh[B::SMEM];
+  __shared__ float sums[B::ROWS];
+  const long long row0 = (long long)blockIdx.x * B::ROWS;
+  B b;
+  b.load(z, row0, rows, cols);
+  b.exponentials(cols);
+  b.add_rows(cols, sh, sums, [&](int n, int q) { return b.v[n][q]; });
+  B::each(cols, [&](int n, int q, int col) {
+    const int r = B::group_row(n);
+    if (row0 + r < rows) y[(row0 + r) * cols + col] = b.v[n][q] / sums[r];
+  });
+}
+
+__global__ __launch_bounds__(kRowThreads) void softmax_long_rows_kernel(const float* z, float* y, long long rows,
+                                                                        long long cols) {
+  __shared__ __attribute__((aligned(16))) float sh[kLongRows * kLongPitch];
+  const long long i = (long long)blockIdx.x * kLongRows + (threadIdx.x >> 6);
+  const bool in = i < rows;
+  const float* row = z + min(i, rows - 1) * cols;
+  const float mx = wave_max_row(row, cols);
+  const float sum = long_row_sum(cols, in, sh, [&](long long j) { return expf(row[j] - mx); });
+  if (in)
+    for (long long j = threadIdx.x & 63; j < cols; j += 64) y[i * cols + j] = expf(row[j] - mx) / sum;
+}
+
+// ops.rs:291-309: dx = s ⊙ (g − Σ_j g_j s_j), per row.  dx may be s or g.
+template <class B>
+__global__ __launch_bounds__(B::T) void softmax_rows_vjp_kernel(const float* s, const float* g, float* dx,
+                                                                long long rows, int cols) {
+  __shared__ __attribute__((aligned(16))) float sh[B::SMEM];
+  __shared__ float sums[B::ROWS];
+  const long long row0 = (long long)blockIdx.x * B::ROWS;
+  B sb, gb;
+  sb.load(s, row0, rows, cols);
+  gb.load(g, row0, rows, cols);
+  sb.add_rows(cols, sh, sums, [&](int n, int q) { return gb.v[n][q] * sb.v[n][q]; });
+  B::each(cols, [&](int n, int q, int col) {
+    const int r = B::group_row(n);
+    if (row0 + r < rows) dx[(row0 + r) * cols + col] = sb.v[n][q] * (gb.v[n][q] - sums[r]);
+  });
+}
+
+__global__ __launch_bounds__(kRowThreads) void softmax_long_rows_vjp_kernel(const float* s, const float* g, float* dx,
+                                                                            long long rows, long long cols) {
+  __shared__ __attribute__((aligned(16))) float sh[kLongRows * kLongPitch];
+  const long long i = (long long)blockIdx.x * kLongRows + (threadIdx.x >> 6);
+  const bool in = i < rows;
+  const float* sr = s + min(i, rows - 1) * cols;
+  const float* gr = g + min(i, rows - 1) * cols;
+  const float dot = long_row_sum(cols, in, sh, [&](long long j) { return gr[j] * sr[j]; });
+  if (in)
+    for (long long j = threadIdx.x & 63; j < cols; j += 64) dx[i * cols + j] = sr[j] * (gr[j] - dot);
 }
 
 // Per-element loss terms (summed by the two-stage sum) and the unscaled
@@ -263,48 +446,92 @@ __global__ __launch_bounds__(256) void loss_terms_kernel(int kind, const float* 
   }
 }
 
-// losses.rs:99-115 from the logits in one pass per row (one thread per row):
-// the softmax of tensor.rs:455-472 (max, exp into dir, sequential sum,
-// divide), then dir = p − y and the row's loss terms −y·ln(max(p, 1e-12))
-// (y ≠ 0) added in column order.  The row sums are added by a block tree;
-// with one block the launch also writes value = (0 + total) / div, else each
-// block writes its part for sum_stage2.
-__global__ __launch_bounds__(256) void xent_logits_kernel(const float* __restrict__ z, const float* __restrict__ y,
-                                                          float* __restrict__ dir, long long rows, long long cols,
-                                                          float* __restrict__ part, float div,
-                                                          float* __restrict__ out, float dir_scale) {
-  __shared__ float sh[256];
-  const long long i = blockIdx.x * 256LL + threadIdx.x;
-  float row_term = 0.0f;
-  if (i < rows) {
-    const float* zr = z + i * cols;
-    const float* yr = y + i * cols;
-    float* d = dir + i * cols;
-    float mx = -INFINITY;
-    for (long long j = 0; j < cols; ++j) mx = fmaxf(mx, zr[j]);
-    float sum = 0.0f;
-    for (long long j = 0; j < cols; ++j) {
-      const float e = expf(zr[j] - mx);
-      d[j] = e;
-      sum += e;
-    }
-    for (long long j = 0; j < cols; ++j) {
-      const float pj = d[j] / sum, yj = yr[j];
-      if (yj != 0.0f) row_term += -(yj * logf(fmaxf(pj, 1e-12f)));
-      d[j] = (pj - yj) * dir_scale;  // dir_scale 1 leaves P − Y exactly as it is
-    }
-  }
-  sh[threadIdx.x] = row_term;
+// losses.rs:99-115 from the logits in one pass per row: the softmax of
+// softmax_rows_kernel (the same bits), then dir = p − y and the row's loss
+// terms −y·ln(max(p, 1e-12)) (y ≠ 0).  Each thread adds its terms, a block
+// tree adds the threads; with one block the launch also writes value =
+// (0 + total) / div, else each block writes its part for sum_stage2.  dir may
+// be z.
+template <int T>
+__device__ inline void loss_block_sum(float terms, float* __restrict__ part, float div, float* __restrict__ out) {
+  __shared__ float red[T];
+  red[threadIdx.x] = terms;
   __syncthreads();
-  for (int w = 128; w > 0; w >>= 1) {
-    if ((int)threadIdx.x < w) sh[threadIdx.x] += sh[threadIdx.x + w];
+  for (int w = T / 2; w > 0; w >>= 1) {
+    if ((int)threadIdx.x < w) red[threadIdx.x] += red[threadIdx.x + w];
     __syncthreads();
   }
   if (threadIdx.x == 0) {
-    if (gridDim.x == 1) out[0] = (0.0f + sh[0]) / div;
-    else part[blockIdx.x] = sh[0];
+    if (gridDim.x == 1) out[0] = (0.0f + red[0]) / div;
+    else part[blockIdx.x] = red[0];
   }
 }
+
+// dir_scale 1 leaves P − Y exactly as it is.
+__device__ inline float xent_element(float p, float y, float dir_scale, float& terms) {
+  if (y != 0.0f) terms += -(y * logf(fmaxf(p, 1e-12f)));
+  return (p - y) * dir_scale;
+}
+
+template <class B>
+__global__ __launch_bounds__(B::T) void xent_logits_kernel(const float* z, const float* __restrict__ y, float* dir,
+                                                           long long rows, int cols, float* __restrict__ part,
+                                                           float div, float* __restrict__ out, float dir_scale) {
+  __shared__ __attribute__((aligned(16))) float sh[B::SMEM];
+  __shared__ float sums[B::ROWS];
+  const long long row0 = (long long)blockIdx.x * B::ROWS;
+  B zb, yb;
+  zb.load(z, row0, rows, cols);
+  yb.load(y, row0, rows, cols);
+  zb.exponentials(cols);
+  zb.add_rows(cols, sh, sums, [&](int n, int q) { return zb.v[n][q]; });
+  float terms = 0.0f;
+  B::each(cols, [&](int n, int q, int col) {
+    const int r = B::group_row(n);
+    if (row0 + r < rows)
+      dir[(row0 + r) * cols + col] = xent_element(zb.v[n][q] / sums[r], yb.v[n][q], dir_scale, terms);
+  });
+  loss_block_sum<B::T>(terms, part, div, out);
+}
+
+// Also the form for no rows or no columns (nothing to load): value = 0 / div.
+__global__ __launch_bounds__(kRowThreads) void xent_logits_long_kernel(const float* z, const float* __restrict__ y,
+                                                                       float* dir, long long rows, long long cols,
+                                                                       float* __restrict__ part, float div,
+                                                                       float* __restrict__ out, float dir_scale) {
+  __shared__ __attribute__((aligned(16))) float sh[kLongRows * kLongPitch];
+  const long long i = (long long)blockIdx.x * kLongRows + (threadIdx.x >> 6);
+  const bool in = i < rows;
+  const float* row = z + (in ? i : 0) * cols;
+  const float mx = in ? wave_max_row(row, cols) : 0.0f;
+  const float sum = long_row_sum(cols, in, sh, [&](long long j) { return expf(row[j] - mx); });
+  float terms = 0.0f;
+  if (in)
+    for (long long j = threadIdx.x & 63; j < cols; j += 64) {
+      const long long e = i * cols + j;
+      dir[e] = xent_element(expf(row[j] - mx) / sum, y[e], dir_scale, terms);
+    }
+  loss_block_sum<kRowThreads>(terms, part, div, out);
+}
+
+// f(Band) for rows of 1 <= cols <= 1024: the fewest lanes that hold the row
+// in one register each up to 64 columns (narrow rows fill the lanes with
+// rows), else a wave with 4 or 16 registers.  One row per group: the blocks of
+// a CU then add, load and store beside each other (four rows per group, in a
+// quarter of the blocks, 18.7 + 15.3 us at 4096 x 1000 against N1_US).
+template <class F>
+hipError_t by_row_length(long long cols, F&& f) {
+#define RT_BAND(l, r) return f(Band<l, r, 1, kRowThreads>{})
+  if (cols <= 4) RT_BAND(4, 1);
+  if (cols <= 8) RT_BAND(8, 1);
+  if (cols <= 16) RT_BAND(16, 1);
+  if (cols <= 32) RT_BAND(32, 1);
+  if (cols <= 64) RT_BAND(64, 1);
+  if (cols <= 256) RT_BAND(64, 4);
+  RT_BAND(64, 16);
+#undef RT_BAND
+}
+constexpr long long kBandCols = 1024;
 
 unsigned grid_for(long long n) { return (unsigned)std::max<long long>(1, std::min<long long>((n + 255) / 256, 8192)); }
 
@@ -426,7 +653,7 @@ hipError_t sum_all_launch(hipStream_t s, const float* x, long long n, float div,
   const long long parts = (long long)sum_scratch_elems(n);
   const long long chunk = std::max<long long>(1, (n + parts - 1) / parts);
   rt::launch(sum_stage1, dim3((unsigned)parts), dim3(256), 0, s, x, n, chunk, scratch, div, out);
-  if (parts > 1) rt::launch(sum_stage2, dim3(1), dim3(64), 0, s, scratch, (int)parts, div, out);
+  if (parts > 1) rt::launch(sum_stage2, dim3(1), dim3(256), 0, s, scratch, (int)parts, div, out);
   return hipGetLastError();
 }
 
@@ -436,29 +663,78 @@ hipError_t scalar_fill_launch(hipStream_t s, const float* scalar, float div, con
   return hipGetLastError();
 }
 
+static dim3 band_grid(long long rows, int per) { return dim3((unsigned)((rows + per - 1) / per)); }
+
 hipError_t softmax_rows_launch(hipStream_t s, const float* z, float* y, long long rows, long long cols) {
-  if (rows <= 0) return hipSuccess;
-  rt::launch(softmax_rows_kernel, dim3((unsigned)((rows + 255) / 256)), dim3(256), 0, s, z, y, rows, cols);
-  return hipGetLastError();
+  if (rows <= 0 || cols <= 0) return hipSuccess;
+  if (cols > kBandCols) {
+    rt::launch(softmax_long_rows_kernel, band_grid(rows, kLongRows), dim3(kRowThreads), 0, s, z, y, rows, cols);
+    return hipGetLastError();
+  }
+  return by_row_length(cols, [&](auto band) {
+    using B = decltype(band);
+    rt::launch(softmax_rows_kernel<B>, band_grid(rows, B::ROWS), dim3(B::T), 0, s, z, y, rows, (int)cols);
+    return hipGetLastError();
+  });
 }
 
 hipError_t softmax_rows_vjp_launch(hipStream_t s, const float* sm, const float* g, float* dx, long long rows,
                                    long long cols) {
-  if (rows <= 0) return hipSuccess;
-  rt::launch(softmax_rows_vjp_kernel, dim3((unsigned)((rows + 255) / 256)), dim3(256), 0, s, sm, g, dx, rows,
-                     cols);
-  return hipGetLastError();
+  if (rows <= 0 || cols <= 0) return hipSuccess;
+  if (cols > kBandCols) {
+    rt::launch(softmax_long_rows_vjp_kernel, band_grid(rows, kLongRows), dim3(kRowThreads), 0, s, sm, g, dx, rows,
+               cols);
+    return hipGetLastError();
+  }
+  return by_row_length(cols, [&](auto band) {
+    using B = decltype(band);
+    rt::launch(softmax_rows_vjp_kernel<B>, band_grid(rows, B::ROWS), dim3(B::T), 0, s, sm, g, dx, rows, (int)cols);
+    return hipGetLastError();
+  });
+}
+
+// f(Band or void*) as the loss launch takes it: one block of kLossThreads for
+// a batch of narrow rows that fits it (a second launch, for the parts, costs
+// more: 256 x 10 takes XS_US us), long or empty rows as null.
+template <class F>
+static hipError_t by_loss_shape(long long rows, long long cols, F&& f) {
+  if (rows <= 0 || cols <= 0 || cols > kBandCols) return f(static_cast<void*>(nullptr));
+  if (cols <= 16 && rows <= 256) return f(Band<16, 1, 4, kLossThreads>{});
+  return by_row_length(cols, f);
+}
+
+size_t xent_logits_parts(long long rows, long long cols) {
+  size_t n = 1;
+  (void)by_loss_shape(rows, cols, [&](auto band) {
+    using B = decltype(band);
+    if constexpr (std::is_pointer_v<B>) n = (size_t)std::max<long long>(1, (rows + kLongRows - 1) / kLongRows);
+    else n = band_grid(rows, B::ROWS).x;
+    return hipSuccess;
+  });
+  return n;
 }
 
 hipError_t xent_logits_launch(hipStream_t s, const float* z, const float* y, float* dir, long long rows,
                               long long cols, float div, float* out, float* scratch, size_t scratch_elems,
                               float dir_scale) {
-  const long long blocks = std::max<long long>(1, (rows + 255) / 256);
-  if (blocks > 1 && (size_t)blocks > scratch_elems) return hipErrorInvalidValue;
-  rt::launch(xent_logits_kernel, dim3((unsigned)blocks), dim3(256), 0, s, z, y, dir, rows, cols, scratch, div,
-                     out, dir_scale);
-  if (blocks > 1) rt::launch(sum_stage2, dim3(1), dim3(64), 0, s, scratch, (int)blocks, div, out);
-  return hipGetLastError();
+  const size_t blocks = xent_logits_parts(rows, cols);
+  if (blocks > 1 && blocks > scratch_elems) return hipErrorInvalidValue;
+  const dim3 grid((unsigned)blocks);
+  hipError_t e = by_loss_shape(rows, cols, [&](auto band) {
+    using B = decltype(band);
+    if constexpr (std::is_pointer_v<B>)
+      rt::launch(xent_logits_long_kernel, grid, dim3(kRowThreads), 0, s, z, y, dir, rows, cols, scratch, div, out,
+                 dir_scale);
+    else
+      rt::launch(xent_logits_kernel<B>, grid, dim3(B::T), 0, s, z, y, dir, rows, (int)cols, scratch, div, out,
+                 dir_scale);
+    return hipGetLastError();
+  });
+  if (e == hipSuccess && blocks > 1) {
+    rt::launch(sum_stage2, dim3(1), dim3(256), 0, s, scratch, (int)blocks, div, out);
+    e = hipGetLastError();
+  }
+  return e;
 }
 
 hipError_t loss_terms_launch(hipStream_t s, int kind, const float* p, const float* y, float* term, float* dir,
@@ -676,8 +952,7 @@ int rt_loss(rt_ctx* c, rt_loss_kind kind, const rt_buf* p, const rt_buf* y, rt_b
       return fail(c, RT_ERR_SHAPE, "logits and targets differ in shape");  // losses.rs:100
     if (!dir) return fail(c, RT_ERR_INVALID, "the logits form writes dir (it holds the softmax on the way)");
     const long long rows = (long long)p->shape[0], cols = (long long)p->shape[1];
-    const size_t blocks = (size_t)std::max<long long>(1, (rows + 255) / 256);
-    int rc = ensure_scratch(c, blocks);
+    int rc = ensure_scratch(c, xent_logits_parts(rows, cols));
     if (rc) return rc;
     Launch L(c, "loss");
     HIP_TRY(c,
