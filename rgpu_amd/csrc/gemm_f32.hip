@@ -1,4 +1,4 @@
-// f32 GEMM on CDNA4 matrix cores: v_mfma_f32_16x16x4_f32, f32 accumulate.
+// f32 GEMM on CDNA4 matrix cores.
 //
 // Replaces rtensor's MM_FAST / MM_EPILOGO / MM_SPLITK WGSL kernels
 // (crates/rtensor/src/gpu/gemm.rs:65-494, splitk.rs:33-237) for the three
@@ -7,28 +7,19 @@
 //   TN  C = Aᵀ·B     A [K,M] (M contiguous),  B [K,N] (N contiguous)  dW = Xᵀ·δ
 //   NT  C = A·Bᵀ     A [M,K] (K contiguous),  B [N,K] (K contiguous)  dX = δ·Wᵀ
 //
-// Block = 256 threads = 4 wave64s in a 2x2 arrangement; block tile BM x BN,
-// K staged through LDS 32 at a time, double-buffered with register staging
-// (one barrier per K step).  Each wave owns a (BM/2) x (BN/2) tile made of
-// TM x TN MFMA 16x16 tiles.
-//
-// Lane/element mapping.  A 16x16x4 MFMA takes, in lane l = 16g + r, the A
-// value (row r, k g) and the B value (k g, col r), and returns D(4g+q, r) in
-// accumulator register q.  Rows, columns and k inside a wave tile may be
-// permuted freely as long as A and B agree on k, so:
-//   * MFMA row r of row-tile t is wave row TM*r + t, MFMA col r of col-tile u
-//     is wave col TN*r + u: a lane's TM (TN) rows (cols) are adjacent, so one
-//     LDS vector read serves all of its tiles when the operand is M (N)
-//     contiguous, and the lane finally owns 4*TM adjacent rows x TN adjacent
-//     columns of C (vector stores along N);
-//   * within a 16-wide k chunk, MFMA step s of lane group g uses k = 4g + s,
-//     so a lane's 4 steps are adjacent k when the operand is K contiguous (one
-//     LDS vector read serves all four steps).
+// Five kernels share the work (dispatch_tile):
+//   F32Split    f32 by exact splits on the bf16 matrix units: most products
+//   F32Dma      v_mfma_f32_16x16x4_f32 fed by direct-to-LDS loads: whole 64x64
+//               tiles over a short K (dma_better)
+//   F32Tile     the same MFMA, register-staged, any shape: weight gradients
+//               over at most 128 rows (row_order_tn)
+//   F32RankK    dX of a narrow layer (K <= 16)
+//   gemm_f32_skinny_kernel   at most 64 rows of output
 //
 // Epilogues run on the accumulators in registers: bias, bias+ReLU (forward,
 // mm_bias in gemm.rs:452-493) and the ReLU mask (δ ← acc ⊙ 1[A>0], fusing
 // RELU_BWD, kernels.rs:119-131).  For TN with a colsum target the blocks of
-// the first M tile also sum the B tiles they stage in LDS over K: that is
+// the first M tile also sum the B values they stage over K: that is
 // db = 1ᵀ·δ (COLSUM, kernels.rs:182-199) at no extra HBM traffic.
 // With more than one K slice, each slice writes a raw f32 partial plane and
 // splitk_reduce sums the planes in slice order (REDUZ, splitk.rs:240-256):
@@ -91,40 +82,37 @@ __device__ inline f4 load4(const float* base, int ld, int row, int col, int rows
 }
 
 // One block's work: tile `bid` (already XCD-renumbered, in [0, tiles)) of
-// K slice `split`.
+// K slice `split`, with v_mfma_f32_16x16x4_f32, every access bounds-checked:
+// short weight gradients (row_order_tn) and operands whose rows are too long
+// for the tiles below.
 //
-// The block is KS groups of 2x2 waves.  Every group computes the whole
-// BM x BN tile, each over its own share of every BK-wide K step (SUB
-// sub-steps of 16), and at the end the groups' accumulators are summed
-// through LDS in group order.  More waves per tile hide more load latency
-// without shrinking the tile.  PF is how many K steps ahead the global loads
-// run: 1 (one register stage) or 2 (two register stages, alternating).
-template <int BM, int BN, bool A_KC, bool B_KC, int BK = 32, int KS = 1, int PF = 1>
+// Four wave64s in a 2x2 arrangement, K staged through LDS 32 at a time,
+// double-buffered with register staging (one barrier per K step).  A 16x16x4
+// MFMA takes, in lane l = 16g + r, the A value (row r, k g) and the B value
+// (k g, col r), and returns D(4g+q, r) in accumulator register q.  Rows,
+// columns and k inside a wave tile may be permuted freely as long as A and B
+// agree on k, so MFMA row r of row-tile t is wave row TM*r + t (likewise the
+// columns), and within a 16-wide k chunk MFMA step s of lane group g uses k =
+// 4g + s: one LDS vector read serves a lane's tiles or steps.
+template <bool A_KC, bool B_KC>
 struct F32Tile {
-  static constexpr int THREADS = 256 * KS;
+  static constexpr int THREADS = 256, BM = 64, BN = 64, BK = 32;
   static constexpr int PAD = 4;
   static constexpr int TM = BM / 32, TN = BN / 32;  // MFMA tiles per wave (2x2 waves of BM/2 x BN/2)
   static constexpr int A_STRIDE = A_KC ? (BK + PAD) : (BM + PAD);
   static constexpr int B_STRIDE = B_KC ? (BK + PAD) : (BN + PAD);
   static constexpr int A_ELEMS = A_KC ? BM * A_STRIDE : BK * A_STRIDE;
   static constexpr int B_ELEMS = B_KC ? BN * B_STRIDE : BK * B_STRIDE;
-  static constexpr int PIPE = 2 * (A_ELEMS + B_ELEMS);  // floats: two stages of both operands
-  static constexpr int RED = (KS - 1) * BM * BN;        // floats: accumulators of groups 1..KS-1
-  static constexpr int SMEM = PIPE > RED ? PIPE : RED;
-  static constexpr int A_LD = BM * BK / 4 / THREADS;  // float4 loads per thread per K step
+  static constexpr int SMEM = 2 * (A_ELEMS + B_ELEMS);  // floats: two stages of both operands
+  static constexpr int A_LD = BM * BK / 4 / THREADS;    // float4 loads per thread per K step
   static constexpr int B_LD = BN * BK / 4 / THREADS;
-  static constexpr int SUB = BK / 16 / KS;
-  static_assert(BM % 32 == 0 && BN % 32 == 0 && BM <= 128 && BN <= 128, "tile");
-  static_assert(A_LD >= 1 && B_LD >= 1 && BM * BK % (4 * THREADS) == 0 && BN * BK % (4 * THREADS) == 0,
-                "tile loads must split evenly over the threads");
-  static_assert(SUB >= 1 && BK % (16 * KS) == 0, "each group takes whole 16-wide sub-steps");
-  static_assert(PF == 1 || PF == 2, "prefetch depth");
+  static constexpr int SUB = BK / 16;
 
   __device__ static void run(const F32Args& p, int bid, int split, float* smem);
 };
 
-template <int BM, int BN, bool A_KC, bool B_KC, int BK, int KS, int PF>
-__device__ void F32Tile<BM, BN, A_KC, B_KC, BK, KS, PF>::run(const F32Args& p, int bid, int split, float* smem) {
+template <bool A_KC, bool B_KC>
+__device__ void F32Tile<A_KC, B_KC>::run(const F32Args& p, int bid, int split, float* smem) {
   float* const sA0 = smem;
   float* const sB0 = smem + 2 * A_ELEMS;
   auto sA = [&](int buf) { return sA0 + buf * A_ELEMS; };
@@ -132,9 +120,8 @@ __device__ void F32Tile<BM, BN, A_KC, B_KC, BK, KS, PF>::run(const F32Args& p, i
 
   const int tid = threadIdx.x;
   const int lane = tid & 63, wave = tid >> 6;
-  const int kg = wave >> 2, wq = wave & 3;  // K group, wave within the group
   const int g = lane >> 4, r = lane & 15;
-  const int wm = (wq >> 1) * (BM / 2), wn = (wq & 1) * (BN / 2);
+  const int wm = (wave >> 1) * (BM / 2), wn = (wave & 1) * (BN / 2);
 
   constexpr int GROUP = 8;
   const int per_group = GROUP * p.tiles_n;
@@ -209,8 +196,7 @@ __device__ void F32Tile<BM, BN, A_KC, B_KC, BK, KS, PF>::run(const F32Args& p, i
     const float* as = sA(buf);
     const float* bs = sB(buf);
 #pragma unroll
-    for (int s2 = 0; s2 < SUB; ++s2) {
-      const int ss = kg * SUB + s2;
+    for (int ss = 0; ss < SUB; ++ss) {
       float af[TM][4], bf[TN][4];
       if constexpr (A_KC) {
 #pragma unroll
@@ -261,70 +247,21 @@ __device__ void F32Tile<BM, BN, A_KC, B_KC, BK, KS, PF>::run(const F32Args& p, i
   };
 
   if (nk > 0) {
-    if constexpr (PF == 1) {
-      f4 ra[A_LD], rb[B_LD];
-      load_tiles(ra, rb, kb);
-      store_tiles(ra, rb, 0);
+    f4 ra[A_LD], rb[B_LD];
+    load_tiles(ra, rb, kb);
+    store_tiles(ra, rb, 0);
+    __syncthreads();
+    for (int kt = 0; kt < nk; ++kt) {
+      const int cur = kt & 1;
+      if (kt + 1 < nk) load_tiles(ra, rb, kb + (kt + 1) * BK);
+      compute(cur);
+      colsum(cur);
+      if (kt + 1 < nk) store_tiles(ra, rb, cur ^ 1);
       __syncthreads();
-      for (int kt = 0; kt < nk; ++kt) {
-        const int cur = kt & 1;
-        if (kt + 1 < nk) load_tiles(ra, rb, kb + (kt + 1) * BK);
-        compute(cur);
-        colsum(cur);
-        if (kt + 1 < nk) store_tiles(ra, rb, cur ^ 1);
-        __syncthreads();
-      }
-    } else {
-      // Register stage j holds K step kt + j; the loads of step kt + 2 are
-      // issued before step kt computes and stored after step kt + 1 does.
-      f4 ra0[A_LD], rb0[B_LD], ra1[A_LD], rb1[B_LD];
-      load_tiles(ra0, rb0, kb);
-      if (nk > 1) load_tiles(ra1, rb1, kb + BK);
-      store_tiles(ra0, rb0, 0);
-      __syncthreads();
-      auto iter = [&](int kt, f4 (&la)[A_LD], f4 (&lb)[B_LD], const f4 (&sa)[A_LD], const f4 (&sb)[B_LD]) {
-        const int cur = kt & 1;
-        if (kt + 2 < nk) load_tiles(la, lb, kb + (kt + 2) * BK);
-        compute(cur);
-        colsum(cur);
-        if (kt + 1 < nk) store_tiles(sa, sb, cur ^ 1);
-        __syncthreads();
-      };
-      for (int kt = 0; kt < nk; kt += 2) {
-        iter(kt, ra0, rb0, ra1, rb1);
-        if (kt + 1 < nk) iter(kt + 1, ra1, rb1, ra0, rb0);
-      }
     }
   }
 
   if (do_cs && n0 + tid < p.N) p.colsum[(long long)split * p.N + n0 + tid] = cs;
-
-  if constexpr (KS > 1) {
-    // Groups 1.. park their accumulators (the main loop ended on a barrier,
-    // so the pipeline buffers are free); group 0 adds them in group order.
-    constexpr int PER = TM * TN * 4;
-    if (kg > 0) {
-      float* dst = smem + ((kg - 1) * 4 + wq) * PER * 64 + lane;
-#pragma unroll
-      for (int t = 0; t < TM; ++t)
-#pragma unroll
-        for (int u = 0; u < TN; ++u)
-#pragma unroll
-          for (int q = 0; q < 4; ++q) dst[((t * TN + u) * 4 + q) * 64] = acc[t][u][q];
-    }
-    __syncthreads();
-    if (kg > 0) return;
-#pragma unroll
-    for (int j = 1; j < KS; ++j) {
-      const float* src = smem + ((j - 1) * 4 + wq) * PER * 64 + lane;
-#pragma unroll
-      for (int t = 0; t < TM; ++t)
-#pragma unroll
-        for (int u = 0; u < TN; ++u)
-#pragma unroll
-          for (int q = 0; q < 4; ++q) acc[t][u][q] += src[((t * TN + u) * 4 + q) * 64];
-    }
-  }
 
   // Epilogue.  Lane owns rows m0+wm+TM*(4g+q)+t and columns n0+wn+TN*r+u.
   const bool partial = p.splits > 1;
@@ -372,8 +309,436 @@ __device__ void F32Tile<BM, BN, A_KC, B_KC, BK, KS, PF>::run(const F32Args& p, i
   }
 }
 
-// ---------------------------------------------------------------- full-tile kernel
-// For whole 64x64 tiles with 16-byte aligned operands the tiles go from
+// ---------------------------------------------------------------- f32 tile on the bf16 matrix units
+// An f32 value is the exact sum of three bf16 values: hi = bf16(x), mid =
+// bf16(x - hi), lo = bf16(x - hi - mid), each remainder exact in f32 (8 + 8 +
+// 8 significant bits).  A product of two f32 values is then nine bf16
+// products, each exact in the MFMA's f32 accumulator; the three smallest (mid
+// lo, lo mid, lo lo: below 2^-26 of the product, against the 2^-24 that each
+// f32 sum rounds by) are left out, and six v_mfma_f32_16x16x32_bf16 replace
+// eight v_mfma_f32_16x16x4_f32 at 16 times their rate.  The bf16 MFMA keeps
+// subnormals, so the split holds down to |x| ~ 2^-109.
+//
+// Block: 256 threads, 4 waves stacked along M, each 16 TM rows by all BN =
+// 16 TN columns.  A wave loads its own A rows straight into registers in
+// fragment order (nothing shares them) and splits them there; B, which all
+// four waves read, is loaded by the block, split once and put into LDS as
+// three bf16 planes [col][32 k] (16-byte granule j of column c at j ^ ((c >>
+// 2) & 3): conflict-free reads and writes).  Global loads run two K stages of
+// 32 ahead, the split one stage ahead, one barrier per stage.  MFMAs take the
+// operands swapped, so lane (g, r) ends with C(row 16t + r, columns 16u + 4g
+// .. + 3): float4 stores.
+//
+// A result that is not finite (an operand was not, or a sum overflowed) says
+// nothing about which: inf - inf in the split, or inf times a zero part.  A
+// wave that sees one computes its tile again with the f32 MFMA.
+typedef __bf16 b2 __attribute__((ext_vector_type(2)));
+typedef __bf16 b8 __attribute__((ext_vector_type(8)));
+typedef unsigned int u4 __attribute__((ext_vector_type(4)));
+
+// The two selectors of split8's remainders: dot2(hi pair, {-1, 0}) + x0.
+// Held in registers: as literals they were encoded into the instruction with
+// the halves exchanged.
+struct SplitSel {
+  b2 first, second;
+  __device__ inline SplitSel() {
+    first = b2{(__bf16)-1.0f, (__bf16)0.0f};
+    second = b2{(__bf16)0.0f, (__bf16)-1.0f};
+    asm volatile("" : "+v"(first), "+v"(second));
+  }
+};
+
+// Eight f32 values into their three bf16 planes, 7 VALU instructions a pair,
+// in 14 steps of two: step Q of the eight values x (overwritten by their
+// remainders).  Breadth first, so that no step needs the result of the one
+// before it.
+constexpr int kSplitSteps = 14;
+template <int Q>
+__device__ __forceinline__ void split_step(float (&x)[8], const SplitSel& sel, u4 (&out)[3]) {
+  constexpr int plane = Q < 6 ? 0 : Q < 12 ? 1 : 2, q = Q % 6;
+  if constexpr (q < 2) {
+#pragma unroll
+    for (int i = 2 * q; i < 2 * q + 2; ++i)
+      out[plane][i] = __builtin_bit_cast(unsigned, __builtin_convertvector((f2{x[2 * i], x[2 * i + 1]}), b2));
+  } else {
+    constexpr int i = q - 2;
+    const b2 h = __builtin_bit_cast(b2, (unsigned)out[plane][i]);
+    x[2 * i] = __builtin_amdgcn_fdot2_f32_bf16(h, sel.first, x[2 * i], false);
+    x[2 * i + 1] = __builtin_amdgcn_fdot2_f32_bf16(h, sel.second, x[2 * i + 1], false);
+  }
+}
+
+// A tile's plain stores (F32Split::run's default epilogue).
+struct NoEpi {
+  static constexpr bool kOn = false;
+};
+
+template <int TM_, int TN_, bool A_KC, bool B_KC>
+struct F32Split {
+  static constexpr int TM = TM_, TN = TN_;
+  static constexpr int THREADS = 256, BM = 64 * TM, BN = 16 * TN, BK = 64, KK = BK / 32;
+  static constexpr int PLANE = BN * BK;             // halves
+  static constexpr int SMEM = 2 * 3 * PLANE / 2;    // floats: two stages of three planes
+  static constexpr int UNITS = BN * BK / 8;         // (column, 8-k granule) units of B per stage
+  static constexpr int UPT = UNITS / THREADS;
+  static constexpr bool CS = !A_KC && !B_KC;  // column sums of B: TN only
+  static_assert(TN % 2 == 0 && UNITS % THREADS == 0, "tile");
+
+  template <class Epi = NoEpi>
+  __device__ static void run(const F32Args& p, int bid, int split, float* smem, const Epi& e = Epi{});
+  __device__ static void plain_f32(const F32Args& p, f4 (&acc)[TM][TN], int row0, int n0, int kb, int ke, int g,
+                                   int r);
+  // The k that element e of granule j stands for within a stage.  An MFMA may
+  // take its 32 k in any order as long as A and B agree; this one makes the
+  // 16-byte loads of four neighbouring granules of a row contiguous.
+  __device__ static constexpr int k_of(int j, int e) { return 32 * (j / 4) + 4 * (j % 4) + (e < 4 ? e : 12 + e); }
+  // Place of granule j (8 k) of column c in an LDS plane (halves).
+  __device__ static inline int place(int c, int j) { return c * BK + 8 * (j ^ ((c >> 1) & 7)); }
+};
+
+__device__ inline bool finite4(const f4& v) {
+  return fabsf(v[0]) <= 3.402823466e38f && fabsf(v[1]) <= 3.402823466e38f && fabsf(v[2]) <= 3.402823466e38f &&
+         fabsf(v[3]) <= 3.402823466e38f;
+}
+
+// The wave's tile with v_mfma_f32_16x16x4_f32, operands element by element
+// from memory (zero outside): only for tiles that came out non-finite.
+template <int TM, int TN, bool A_KC, bool B_KC>
+__device__ __forceinline__ void F32Split<TM, TN, A_KC, B_KC>::plain_f32(const F32Args& p, f4 (&acc)[TM][TN], int row0,
+                                                                        int n0, int kb, int ke, int g, int r) {
+#pragma unroll
+  for (int t = 0; t < TM; ++t)
+#pragma unroll
+    for (int u = 0; u < TN; ++u) acc[t][u] = f4{0.0f, 0.0f, 0.0f, 0.0f};
+  for (int k0 = kb; k0 < ke; k0 += 4) {
+    const int k = k0 + g;
+    float a[TM], b[TN];
+#pragma unroll
+    for (int t = 0; t < TM; ++t) {
+      const int m = row0 + 16 * t + r;
+      a[t] = k < ke && m < p.M ? p.A[A_KC ? (long long)m * p.lda + k : (long long)k * p.lda + m] : 0.0f;
+    }
+#pragma unroll
+    for (int u = 0; u < TN; ++u) {
+      const int n = n0 + 16 * u + r;
+      b[u] = k < ke && n < p.N ? p.B[B_KC ? (long long)n * p.ldb + k : (long long)k * p.ldb + n] : 0.0f;
+    }
+#pragma unroll
+    for (int t = 0; t < TM; ++t)
+#pragma unroll
+      for (int u = 0; u < TN; ++u) acc[t][u] = __builtin_amdgcn_mfma_f32_16x16x4f32(b[u], a[t], acc[t][u], 0, 0, 0);
+  }
+}
+
+// Stores of a wave tile: lane (g, r) holds rows row0 + 16t + r, columns n0 +
+// 16u + 4g .. + 3.
+template <int EPI, int TM, int TN>
+__device__ __forceinline__ void store_rows(const F32Args& p, const f4 (&acc)[TM][TN], int row0, int n0, int g, int r,
+                                            int split) {
+  float* C = p.C + (p.splits > 1 ? (long long)split * p.split_stride : 0);
+#pragma unroll
+  for (int t = 0; t < TM; ++t) {
+    const int row = row0 + 16 * t + r;
+    if (row >= p.M) continue;
+    const long long row_off = (long long)row * p.ldc;
+#pragma unroll
+    for (int u = 0; u < TN; ++u) {
+      const int col = n0 + 16 * u + 4 * g;
+      f4 v = acc[t][u];
+      if (p.vec_c && col + 4 <= p.N) {
+        if constexpr (EPI == RT_EPI_BIAS || EPI == RT_EPI_BIAS_RELU) {
+          const f4 b = *reinterpret_cast<const f4*>(p.bias + col);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            v[e] = v[e] + b[e];
+            if constexpr (EPI == RT_EPI_BIAS_RELU) v[e] = fmaxf(v[e], 0.0f);
+          }
+        } else if constexpr (EPI == RT_EPI_RELU_MASK) {
+          const f4 mk = *reinterpret_cast<const f4*>(p.mask + row_off + col);
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            if (!(mk[e] > 0.0f)) v[e] = 0.0f;
+        }
+        *reinterpret_cast<f4*>(C + row_off + col) = v;
+        continue;
+      }
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        if (col + e >= p.N) break;
+        float x = v[e];
+        if constexpr (EPI == RT_EPI_BIAS || EPI == RT_EPI_BIAS_RELU) {
+          x = x + p.bias[col + e];
+          if constexpr (EPI == RT_EPI_BIAS_RELU) x = fmaxf(x, 0.0f);
+        } else if constexpr (EPI == RT_EPI_RELU_MASK) {
+          if (!(p.mask[row_off + col + e] > 0.0f)) x = 0.0f;
+        }
+        C[row_off + col + e] = x;
+      }
+    }
+  }
+}
+
+template <int TM, int TN, class Epi>
+__device__ __forceinline__ void store_tile(const F32Args& p, const f4 (&acc)[TM][TN], int row0, int n0, int g, int r,
+                                           int split, const Epi& e) {
+  if constexpr (Epi::kOn) return e.tile(p, acc, row0, n0, g, r);
+  if (p.splits > 1) return store_rows<RT_EPI_NONE>(p, acc, row0, n0, g, r, split);
+  switch (p.epi) {
+    case RT_EPI_BIAS: return store_rows<RT_EPI_BIAS>(p, acc, row0, n0, g, r, split);
+    case RT_EPI_BIAS_RELU: return store_rows<RT_EPI_BIAS_RELU>(p, acc, row0, n0, g, r, split);
+    case RT_EPI_RELU_MASK: return store_rows<RT_EPI_RELU_MASK>(p, acc, row0, n0, g, r, split);
+    default: return store_rows<RT_EPI_NONE>(p, acc, row0, n0, g, r, split);
+  }
+}
+
+template <int TM, int TN, bool A_KC, bool B_KC>
+template <class Epi>
+__device__ void F32Split<TM, TN, A_KC, B_KC>::run(const F32Args& p, int bid, int split, float* smem, const Epi& e) {
+  unsigned short* const lds = reinterpret_cast<unsigned short*>(smem);
+  const int tid = threadIdx.x;
+  const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int g = lane >> 4, r = lane & 15;
+
+  constexpr int GROUP = 8;
+  const int per_group = GROUP * p.tiles_n;
+  const int grp = bid / per_group;
+  const int first_m = grp * GROUP;
+  const int gsize = min(p.tiles_m - first_m, GROUP);
+  const int in_grp = bid - grp * per_group;
+  const int tile_m = first_m + in_grp % gsize;
+  const int tile_n = in_grp / gsize;
+  const int m0 = tile_m * BM, n0 = tile_n * BN;
+  const int row0 = m0 + 16 * TM * wave;
+
+  const int kb = split * p.k_per_split;
+  const int ke = min(p.K, kb + p.k_per_split);
+  const int nk = ke > kb ? (ke - kb + BK - 1) / BK : 0;
+
+  // Byte offsets of this lane's loads from the stage's origin (below 2^31,
+  // checked by the host).  Rows and columns past the edge read the last one;
+  // what they give is not stored.
+  int va[TM];
+#pragma unroll
+  for (int t = 0; t < TM; ++t) {
+    const int m = min(row0 + 16 * t + r, p.M - 1) - m0;
+    va[t] = A_KC ? 4 * (m * p.lda + 4 * g) : 4 * (4 * g * p.lda + m);
+  }
+  const int a_kk = A_KC ? 4 * 32 : 4 * 32 * p.lda;  // bytes between the two 32-k steps
+  int vb[UPT], lb[UPT];                             // ... and the unit's place in an LDS plane
+#pragma unroll
+  for (int i = 0; i < UPT; ++i) {
+    const int q = tid + THREADS * i;
+    const int col = B_KC ? q / (BK / 8) : q % BN, j = B_KC ? q % (BK / 8) : q / BN;
+    const int n = min(n0 + col, p.N - 1) - n0;
+    vb[i] = B_KC ? 4 * (n * p.ldb + k_of(j, 0)) : 4 * (k_of(j, 0) * p.ldb + n);
+    lb[i] = place(col, j);
+  }
+
+  // K runs over the stages 0 .. nk - 1; when K is not a multiple of 64 the
+  // remainder is stage 0, so that every load inside the loop is a whole one
+  // (a branch there would make the compiler wait for loads still in flight).
+  const int rest = (ke - kb) % BK;
+  float fa[TM][KK][8], fb[UPT][8];
+  auto rsrcs = [&](int k0, __amdgpu_buffer_rsrc_t& ra, __amdgpu_buffer_rsrc_t& rb) {
+    ra = rt_dev::raw_rsrc(A_KC ? p.A + (long long)m0 * p.lda + k0 : p.A + (long long)k0 * p.lda + m0);
+    rb = rt_dev::raw_rsrc(B_KC ? p.B + (long long)n0 * p.ldb + k0 : p.B + (long long)k0 * p.ldb + n0);
+  };
+  // The f32 values of whole stage s: B's units and the A rows of its first
+  // 32 k (part 0), the A rows of its second 32 k (part 1).
+  auto load_op = [&](const __amdgpu_buffer_rsrc_t& rs, int vo, int so, int ld, auto kc, float (&x)[8]) {
+    if constexpr (decltype(kc)::value) {
+      const u4 lo = __builtin_amdgcn_raw_buffer_load_b128(rs, vo, so, 0);
+      const u4 hi = __builtin_amdgcn_raw_buffer_load_b128(rs, vo, so + 64, 0);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        x[j] = __uint_as_float(lo[j]);
+        x[4 + j] = __uint_as_float(hi[j]);
+      }
+    } else {
+#pragma unroll
+      for (int j = 0; j < 8; ++j)
+        x[j] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rs, vo, so + 4 * k_of(0, j) * ld, 0));
+    }
+  };
+  auto load = [&](int s, auto part) {
+    constexpr int kk = decltype(part)::value;
+    __amdgpu_buffer_rsrc_t ra, rb;
+    rsrcs(kb + s * BK - (rest ? BK - rest : 0), ra, rb);
+    if constexpr (kk == 0) {
+#pragma unroll
+      for (int i = 0; i < UPT; ++i) load_op(rb, vb[i], 0, p.ldb, std::integral_constant<bool, B_KC>{}, fb[i]);
+    }
+#pragma unroll
+    for (int t = 0; t < TM; ++t)
+      load_op(ra, va[t], kk * a_kk, p.lda, std::integral_constant<bool, A_KC>{}, fa[t][kk]);
+  };
+  // The remainder's first k is kb: element by element, zero past it.
+  auto load_rest = [&]() {
+    __amdgpu_buffer_rsrc_t ra, rb;
+    rsrcs(kb, ra, rb);
+    auto at = [](const __amdgpu_buffer_rsrc_t& rs, int off, bool in) {
+      return in ? __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rs, off, 0, 0)) : 0.0f;
+    };
+#pragma unroll
+    for (int i = 0; i < UPT; ++i) {
+      const int q = tid + THREADS * i, gr = B_KC ? q % (BK / 8) : q / BN;
+#pragma unroll
+      for (int j = 0; j < 8; ++j) fb[i][j] = at(rb, vb[i] + 4 * k_of(0, j) * (B_KC ? 1 : p.ldb), k_of(gr, j) < rest);
+    }
+#pragma unroll
+    for (int t = 0; t < TM; ++t)
+#pragma unroll
+      for (int kk = 0; kk < KK; ++kk)
+#pragma unroll
+        for (int j = 0; j < 8; ++j)
+          fa[t][kk][j] = at(ra, va[t] + kk * a_kk + 4 * k_of(0, j) * (A_KC ? 1 : p.lda), k_of(4 * kk + g, j) < rest);
+  };
+
+  // Bias gradient (TN with a colsum target, first M tile): a unit's values are
+  // 8 k rows of one column; they are added in f32, and the column's units in
+  // order at the end.
+  const bool do_cs = CS && p.colsum != nullptr && tile_m == 0;  // uniform over the block
+  float cs[UPT];
+#pragma unroll
+  for (int i = 0; i < UPT; ++i) cs[i] = 0.0f;
+
+  const SplitSel sel;
+  u4 ap[KK][TM][3], bq[3];
+  // Step w of the split of B's units (w / 14), whose planes go to LDS buffer
+  // `buf` as they are complete; likewise of the A rows of one 32-k step.
+  auto split_b = [&](int buf, auto wc) {
+    constexpr int i = decltype(wc)::value / kSplitSteps, q = decltype(wc)::value % kSplitSteps;
+    if constexpr (CS && q == 0) {  // every M tile adds (a branch would part the schedule); the first one stores
+#pragma unroll
+      for (int j = 0; j < 8; ++j) cs[i] += fb[i][j];
+    }
+    split_step<q>(fb[i], sel, bq);
+    if constexpr (q == 1 || q == 7 || q == 13) {  // a plane is complete
+      constexpr int pl = q / 6;
+      *reinterpret_cast<u4*>(&lds[(buf * 3 + pl) * PLANE + lb[i]]) = bq[pl];
+    }
+  };
+  auto split_a = [&](auto kkc, auto wc) {
+    constexpr int kk = decltype(kkc)::value, t = decltype(wc)::value / kSplitSteps;
+    split_step<decltype(wc)::value % kSplitSteps>(fa[t][kk], sel, ap[kk][t]);
+  };
+
+  // The hi·hi products have an accumulator of their own: the small ones, added
+  // into it one MFMA after another, would round it six times per 32 k (which
+  // measured 15% more error than the f32 MFMA on operands after a ReLU).
+  f4 acc[TM][TN], small[TM][TN];
+#pragma unroll
+  for (int t = 0; t < TM; ++t)
+#pragma unroll
+    for (int u = 0; u < TN; ++u) acc[t][u] = small[t][u] = f4{0.0f, 0.0f, 0.0f, 0.0f};
+
+  // (B plane, A plane) of the six products, smallest first.
+  constexpr int PB[6] = {2, 0, 1, 1, 0, 0}, PA[6] = {0, 2, 1, 0, 1, 0};
+  // A stage's MFMAs run over P column pairs (kk, u0); the B fragments of a
+  // pair are read while the pair before it computes.
+  constexpr int P = KK * TN / 2;
+  u4 bp[2][2][3];
+  auto read_pair = [&](int buf, auto ic) {
+    constexpr int i = decltype(ic)::value, kk = i / (TN / 2), u0 = 2 * (i % (TN / 2));
+#pragma unroll
+    for (int uu = 0; uu < 2; ++uu)
+#pragma unroll
+      for (int pl = 0; pl < 3; ++pl)
+        bp[i & 1][uu][pl] = *reinterpret_cast<const u4*>(
+            &lds[(buf * 3 + pl) * PLANE + place(16 * (u0 + uu) + r, 4 * kk + g)]);
+  };
+  using H0 = std::integral_constant<int, 0>;
+  using H1 = std::integral_constant<int, 1>;
+  // The MFMAs of one 32-k step (half a stage), one by one: behind each comes
+  // its share of the `steps` split steps, step(w), and in the middle of a pair
+  // the LDS reads of the next one.  The schedule is fixed here
+  // (sched_barrier): left to itself the compiler puts the splits after the
+  // MFMAs, and with one wave per SIMD nothing else would fill the matrix
+  // unit meanwhile.
+  auto half = [&](int buf, auto hc, auto steps_c, auto&& step) {
+    constexpr int kk = decltype(hc)::value, PH = TN / 2, MF = 12 * TM, SLOTS = PH * MF;
+    constexpr int STEPS = decltype(steps_c)::value;
+    rt_dev::static_for<0, SLOTS>([&](auto sc) {
+      constexpr int slot = decltype(sc)::value, i = kk * PH + slot / MF, m = slot % MF;
+      constexpr int c = m / (2 * TM), uu = m / TM % 2, t = m % TM, u = 2 * (i % PH) + uu;
+      if constexpr (m == MF / 2 && i + 1 < P) read_pair(buf, std::integral_constant<int, i + 1>{});
+      f4& d = c == 5 ? acc[t][u] : small[t][u];
+      d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(b8, bp[i & 1][uu][PB[c]]),
+                                                  __builtin_bit_cast(b8, ap[kk][t][PA[c]]), d, 0, 0, 0);
+      rt_dev::static_for<slot * STEPS / SLOTS, (slot + 1) * STEPS / SLOTS>([&](auto wc) { step(wc); });
+      __builtin_amdgcn_sched_barrier(0);
+    });
+  };
+  constexpr int NA = kSplitSteps * TM, NB = kSplitSteps * UPT;
+
+  if (nk > 0) {
+    if (rest) {
+      load_rest();
+    } else {
+      load(0, H0{});
+      load(0, H1{});
+    }
+    rt_dev::static_for<0, NB>([&](auto wc) { split_b(0, wc); });
+    rt_dev::static_for<0, NA>([&](auto wc) { split_a(H0{}, wc); });
+    rt_dev::barrier_lds();
+    // Stage s: its B planes are in LDS buffer s % 2, the A planes of its
+    // first 32 k in ap[0], the f32 values of its second in fa.  Under the
+    // first half's MFMAs those are split, under the second half's the first
+    // 32 k and B of stage s + 1, fetched at the start of stage s.
+    for (int s = 0; s + 1 < nk; ++s) {
+      const int buf = s & 1;
+      load(s + 1, H0{});
+      read_pair(buf, H0{});
+      __builtin_amdgcn_sched_barrier(0);
+      half(buf, H0{}, std::integral_constant<int, NA>{}, [&](auto wc) { split_a(H1{}, wc); });
+      load(s + 1, H1{});
+      __builtin_amdgcn_sched_barrier(0);
+      half(buf, H1{}, std::integral_constant<int, NA + NB>{}, [&](auto wc) {
+        constexpr int w = decltype(wc)::value;
+        if constexpr (w < NB) split_b(buf ^ 1, wc);
+        else split_a(H0{}, std::integral_constant<int, w - NB>{});
+      });
+      rt_dev::barrier_lds();
+    }
+    const int buf = (nk - 1) & 1;
+    read_pair(buf, H0{});
+    half(buf, H0{}, std::integral_constant<int, NA>{}, [&](auto wc) { split_a(H1{}, wc); });
+    half(buf, H1{}, std::integral_constant<int, 0>{}, [&](auto) {});
+  }
+
+  if (do_cs) {
+    __syncthreads();
+    float* red = smem;  // [granule of 8 k][BN]: the same sums whatever the tile
+#pragma unroll
+    for (int i = 0; i < UPT; ++i) red[tid + THREADS * i] = cs[i];
+    __syncthreads();
+    if (tid < BN && n0 + tid < p.N) {
+      float v = red[tid];
+#pragma unroll
+      for (int j = 1; j < BK / 8; ++j) v += red[j * BN + tid];
+      if constexpr (Epi::kOn)
+        e.bias(p, n0 + tid, v);
+      else
+        p.colsum[(long long)split * p.N + n0 + tid] = v;
+    }
+  }
+
+  bool fine = true;
+#pragma unroll
+  for (int t = 0; t < TM; ++t)
+#pragma unroll
+    for (int u = 0; u < TN; ++u) {
+      acc[t][u] += small[t][u];
+      fine = fine && finite4(acc[t][u]);
+    }
+  if (__any(!fine)) plain_f32(p, acc, row0, n0, kb, ke, g, r);
+
+  store_tile<TM, TN>(p, acc, row0, n0, g, r, split, e);
+}
+
+// ---------------------------------------------------------------- f32 MFMA tile fed by DMA
+// For whole 64x64 tiles over a short K (dma_better) with 16-byte aligned
+// operands the tiles go from
 // global memory straight into LDS (buffer_load ... lds: lane l's 16 bytes
 // land at the instruction's LDS base + 16 l), two stages of BK = 32 k.
 // Within a stage the two 16-k halves are pipelined around one barrier:
@@ -389,11 +754,6 @@ __device__ void F32Tile<BM, BN, A_KC, B_KC, BK, KS, PF>::run(const F32Args& p, i
 //     four k of the lane's four MFMA steps);
 //   M/N-contiguous [k][64]: 64-byte chunk c of row k at c ^ ((k >> 2) & 3); a
 //     fragment is four b32 reads (k = 16 half + 4g + s, column 16u + r).
-// A tile's plain stores (F32Dma::run's default epilogue).
-struct NoEpi {
-  static constexpr bool kOn = false;
-};
-
 struct F32Dma {
   static constexpr int BM = 64, BN = 64, BK = 32, THREADS = 256, WAVES = 4;
   static constexpr int TM = 2, TN = 2;                 // 16x16 MFMA tiles per wave (32x32 wave tile)
@@ -452,35 +812,6 @@ struct F32Dma {
   template <bool A_KC, bool B_KC, class Epi = NoEpi>
   __device__ static void run(const F32Args& p, int bid, int split, float* smem, const Epi& e = Epi{});
 };
-
-template <int EPI>
-__device__ __forceinline__ void f32_store_direct(const F32Args& p, const f4 (&acc)[2][2], int m0, int n0, int wm,
-                                                 int wn, int g, int r, int split) {
-  float* C = p.C + (p.splits > 1 ? (long long)split * p.split_stride : 0);
-#pragma unroll
-  for (int t = 0; t < 2; ++t) {
-    const long long row_off = (long long)(m0 + wm + 16 * t + r) * p.ldc;
-#pragma unroll
-    for (int u = 0; u < 2; ++u) {
-      const int col = n0 + wn + 16 * u + 4 * g;
-      f4 v = acc[t][u];
-      if constexpr (EPI == RT_EPI_BIAS || EPI == RT_EPI_BIAS_RELU) {
-        const f4 b = *reinterpret_cast<const f4*>(p.bias + col);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          v[e] = v[e] + b[e];
-          if constexpr (EPI == RT_EPI_BIAS_RELU) v[e] = fmaxf(v[e], 0.0f);
-        }
-      } else if constexpr (EPI == RT_EPI_RELU_MASK) {
-        const f4 mk = *reinterpret_cast<const f4*>(p.mask + row_off + col);
-#pragma unroll
-        for (int e = 0; e < 4; ++e)
-          if (!(mk[e] > 0.0f)) v[e] = 0.0f;
-      }
-      *reinterpret_cast<f4*>(C + row_off + col) = v;
-    }
-  }
-}
 
 template <bool A_KC, bool B_KC, class Epi>
 __device__ void F32Dma::run(const F32Args& p, int bid, int split, float* smem, const Epi& e) {
@@ -598,29 +929,24 @@ __device__ void F32Dma::run(const F32Args& p, int bid, int split, float* smem, c
     }
   }
 
-  if constexpr (Epi::kOn) return e.tile(p, acc, m0, n0, wm, wn, g, r);
-  if (p.splits > 1) return f32_store_direct<RT_EPI_NONE>(p, acc, m0, n0, wm, wn, g, r, split);
-  switch (p.epi) {
-    case RT_EPI_BIAS: return f32_store_direct<RT_EPI_BIAS>(p, acc, m0, n0, wm, wn, g, r, split);
-    case RT_EPI_BIAS_RELU: return f32_store_direct<RT_EPI_BIAS_RELU>(p, acc, m0, n0, wm, wn, g, r, split);
-    case RT_EPI_RELU_MASK: return f32_store_direct<RT_EPI_RELU_MASK>(p, acc, m0, n0, wm, wn, g, r, split);
-    default: return f32_store_direct<RT_EPI_NONE>(p, acc, m0, n0, wm, wn, g, r, split);
-  }
+  store_tile<TM, TN>(p, acc, m0 + wm, n0 + wn, g, r, split, e);
 }
 
 // Adapter so the single and pair kernels can run an F32Dma layout like an
 // F32Tile.
 template <bool A_KC, bool B_KC>
 struct F32DmaTile {
-  static constexpr int THREADS = F32Dma::THREADS;
-  static constexpr int SMEM = F32Dma::SMEM;
-  __device__ static void run(const F32Args& p, int bid, int split, float* smem) {
-    F32Dma::run<A_KC, B_KC>(p, bid, split, smem);
+  static constexpr int THREADS = F32Dma::THREADS, SMEM = F32Dma::SMEM, BM = F32Dma::BM, BN = F32Dma::BN;
+  template <class Epi = NoEpi>
+  __device__ static void run(const F32Args& p, int bid, int split, float* smem, const Epi& e = Epi{}) {
+    F32Dma::run<A_KC, B_KC>(p, bid, split, smem, e);
   }
 };
 
+// Two waves per SIMD: the compiler would otherwise spread a 128x64 tile over
+// more than half of the registers (4096^3 NN 724 -> 917 us).
 template <class T>
-__global__ __launch_bounds__(T::THREADS) void gemm_f32_kernel(F32Args p) {
+__global__ __launch_bounds__(T::THREADS, 2) void gemm_f32_kernel(F32Args p) {
   __shared__ __attribute__((aligned(16))) float smem[T::SMEM];
   T::run(p, xcd_local(blockIdx.x, gridDim.x), blockIdx.z, smem);
 }
@@ -631,7 +957,7 @@ __global__ __launch_bounds__(T::THREADS) void gemm_f32_kernel(F32Args p) {
 // order, then applies the epilogue.  A rank-K update is a stream of C (and
 // of the mask): the MFMA tile's K pipeline padded to 32 only adds latency.
 struct F32RankK {
-  static constexpr int THREADS = 256;
+  static constexpr int THREADS = 256, BM = 64, BN = 64;
   static constexpr int KMAX = 16;
   static constexpr int LD = KMAX + 1;  // LDS row stride (floats)
   static constexpr int SMEM = 2 * 64 * LD;
@@ -702,7 +1028,7 @@ struct F32RankK {
 // folded into its block range.  n0 is a multiple of 8 so both problems are
 // spread evenly over the XCDs; problem 0 is dispatched first.
 template <class T0, class T1>
-__global__ __launch_bounds__(T0::THREADS) void gemm_f32_pair_kernel(F32Args p0, F32Args p1, int n0) {
+__global__ __launch_bounds__(T0::THREADS, 2) void gemm_f32_pair_kernel(F32Args p0, F32Args p1, int n0) {
   static_assert(T0::THREADS == T1::THREADS, "one block size");
   constexpr int S = T0::SMEM > T1::SMEM ? T0::SMEM : T1::SMEM;
   __shared__ __attribute__((aligned(16))) float smem[S];
@@ -726,7 +1052,7 @@ __global__ __launch_bounds__(T0::THREADS) void gemm_f32_pair_kernel(F32Args p0, 
 // the optimizer blocks of b.  The GEMM is dispatched first; the update, which
 // is HBM-bound, runs on the CUs next to its MFMA-bound tiles.
 template <class T>
-__global__ __launch_bounds__(T::THREADS) void gemm_f32_opt_kernel(F32Args p, rt_opt::OptBatch b, int n_gemm) {
+__global__ __launch_bounds__(T::THREADS, 2) void gemm_f32_opt_kernel(F32Args p, rt_opt::OptBatch b, int n_gemm) {
   static_assert(T::THREADS == rt_opt::kThreads, "one block size");
   __shared__ __attribute__((aligned(16))) float smem[T::SMEM];
   const int blk = blockIdx.x;
@@ -749,34 +1075,32 @@ struct UpdEpi {
   static constexpr bool kOn = true;
   rt::OptTensor w, b;
   rt::OptParams P;
-  __device__ void tile(const F32Args& p, const f4 (&acc)[2][2], int m0, int n0, int wm, int wn, int g,
-                       int r) const {
+  template <int TM, int TN>
+  __device__ void tile(const F32Args& p, const f4 (&acc)[TM][TN], int row0, int n0, int g, int r) const {
     const bool skip = rt_opt::skipped(P);
     const rt_opt::Coef c = rt_opt::coef(P);
     const bool adam = P.kind == 0, has_m = w.m != nullptr;
-    long long idx[2][2];
-#pragma unroll
-    for (int t = 0; t < 2; ++t)
-#pragma unroll
-      for (int u = 0; u < 2; ++u) idx[t][u] = (long long)(m0 + wm + 16 * t + r) * p.ldc + n0 + wn + 16 * u + 4 * g;
+    // Whole tiles only (gemm_opt_update_ok).
+    const long long i0 = (long long)(row0 + r) * p.ldc + n0 + 4 * g;
     // Every load of θ and the state first, so that they go out together
     // (the stores below could alias them as far as the compiler knows).
-    f4 th[2][2], m[2][2], v[2][2];
+    f4 th[TM][TN], m[TM][TN], v[TM][TN];
     if (!skip) {
 #pragma unroll
-      for (int t = 0; t < 2; ++t)
+      for (int t = 0; t < TM; ++t)
 #pragma unroll
-        for (int u = 0; u < 2; ++u) {
-          th[t][u] = *reinterpret_cast<const f4*>(w.theta + idx[t][u]);
-          m[t][u] = has_m ? *reinterpret_cast<const f4*>(w.m + idx[t][u]) : f4{0, 0, 0, 0};
-          v[t][u] = adam ? *reinterpret_cast<const f4*>(w.v + idx[t][u]) : f4{0, 0, 0, 0};
+        for (int u = 0; u < TN; ++u) {
+          const long long i = i0 + (long long)16 * t * p.ldc + 16 * u;
+          th[t][u] = *reinterpret_cast<const f4*>(w.theta + i);
+          m[t][u] = has_m ? *reinterpret_cast<const f4*>(w.m + i) : f4{0, 0, 0, 0};
+          v[t][u] = adam ? *reinterpret_cast<const f4*>(w.v + i) : f4{0, 0, 0, 0};
         }
     }
 #pragma unroll
-    for (int t = 0; t < 2; ++t)
+    for (int t = 0; t < TM; ++t)
 #pragma unroll
-      for (int u = 0; u < 2; ++u) {
-        const long long i = idx[t][u];
+      for (int u = 0; u < TN; ++u) {
+        const long long i = i0 + (long long)16 * t * p.ldc + 16 * u;
         const f4 gv = acc[t][u];
         *reinterpret_cast<f4*>(p.C + i) = gv;
         if (skip) continue;
@@ -805,15 +1129,16 @@ struct UpdEpi {
   }
 };
 
-// gemm_f32_opt_kernel on 64x64 DMA tiles of an unsplit TN product whose
+// gemm_f32_opt_kernel on whole 64x64 tiles of an unsplit TN product whose
 // tiles also update their own layer (UpdEpi).
-__global__ __launch_bounds__(F32Dma::THREADS) void gemm_f32_opt_upd_kernel(F32Args p, rt_opt::OptBatch b, int n_gemm,
-                                                                          UpdEpi u) {
-  static_assert(F32Dma::THREADS == rt_opt::kThreads, "one block size");
-  __shared__ __attribute__((aligned(16))) float smem[F32Dma::SMEM];
+template <class T>
+__global__ __launch_bounds__(T::THREADS, 2) void gemm_f32_opt_upd_kernel(F32Args p, rt_opt::OptBatch b, int n_gemm,
+                                                                        UpdEpi u) {
+  static_assert(T::THREADS == rt_opt::kThreads && T::BM == 64 && T::BN == 64, "one block size, 64x64 tiles");
+  __shared__ __attribute__((aligned(16))) float smem[T::SMEM];
   const int blk = blockIdx.x;
   if (blk < n_gemm) {
-    F32Dma::run<false, false>(p, xcd_local(blk, n_gemm), 0, smem, u);
+    T::run(p, xcd_local(blk, n_gemm), 0, smem, u);
   } else {
     rt_opt::optimizer_block<false>(b, blk - n_gemm);
   }
@@ -822,17 +1147,18 @@ __global__ __launch_bounds__(F32Dma::THREADS) void gemm_f32_opt_upd_kernel(F32Ar
 // Two such products (two layers' dW, each updating its own layer) and the
 // optimizer blocks of b in one launch: blocks [0, n0) problem 0 (n0 a
 // multiple of 8, the padding idle), [n0, n1) problem 1, the rest the update.
-__global__ __launch_bounds__(F32Dma::THREADS) void gemm_f32_opt_upd2_kernel(F32Args p0, F32Args p1, rt_opt::OptBatch b,
-                                                                           int n0, int n1, UpdEpi u0, UpdEpi u1) {
-  static_assert(F32Dma::THREADS == rt_opt::kThreads, "one block size");
-  __shared__ __attribute__((aligned(16))) float smem[F32Dma::SMEM];
+template <class T>
+__global__ __launch_bounds__(T::THREADS, 2) void gemm_f32_opt_upd2_kernel(F32Args p0, F32Args p1, rt_opt::OptBatch b,
+                                                                         int n0, int n1, UpdEpi u0, UpdEpi u1) {
+  static_assert(T::THREADS == rt_opt::kThreads && T::BM == 64 && T::BN == 64, "one block size, 64x64 tiles");
+  __shared__ __attribute__((aligned(16))) float smem[T::SMEM];
   const int blk = blockIdx.x;
   if (blk < n0) {
     const int nb = p0.tiles_m * p0.tiles_n;
     if (blk >= nb) return;  // padding up to a multiple of 8
-    F32Dma::run<false, false>(p0, xcd_local(blk, nb), 0, smem, u0);
+    T::run(p0, xcd_local(blk, nb), 0, smem, u0);
   } else if (blk < n1) {
-    F32Dma::run<false, false>(p1, xcd_local(blk - n0, n1 - n0), 0, smem, u1);
+    T::run(p1, xcd_local(blk - n0, n1 - n0), 0, smem, u1);
   } else {
     rt_opt::optimizer_block<false>(b, blk - n1);
   }
@@ -955,47 +1281,48 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(const float* __restr
   }
 }
 
-template <int BM, int BN, bool A_KC, bool B_KC, int BK = 32, int KS = 1, int PF = 1>
-hipError_t launch_f32(hipStream_t s, F32Args a) {
-  using T = F32Tile<BM, BN, A_KC, B_KC, BK, KS, PF>;
-  a.tiles_m = (a.M + BM - 1) / BM;
-  a.tiles_n = (a.N + BN - 1) / BN;
-  dim3 grid(a.tiles_m * a.tiles_n, 1, a.splits);
-  rt::launch((gemm_f32_kernel<T>), grid, dim3(T::THREADS), 0, s, a);
-  return hipGetLastError();
-}
-
-// 128x128 tiles when they alone give at least two waves of 256 CUs,
-// otherwise 64x64 (4x the workgroups) so small GEMMs still fill the chip;
-// 64x32 for narrow outputs.
-enum TileCfg { kT128, kT64x32, kT64 };
+// Tile of a product: the largest of 128x64, 64x64 and 64x32 that still gives
+// every CU a block (a smaller one splits and reads its operands more often:
+// 4096^3 NN 724 / 821 / 1069 us; too few blocks leave CUs idle: 512x1024, K
+// 2048 in two slices 35.1 / 25.3 / 24.5 us, 300x200, K 500 18.4 / 12.4 / 8.7).
+enum TileCfg { kT128x64, kT64x64, kT64x32 };
 TileCfg pick_tile(const F32Args& a) {
-  const long long t128 = (long long)((a.M + 127) / 128) * ((a.N + 127) / 128) * a.splits;
-  if (t128 >= 512) return kT128;
+  const long long n64 = (a.N + 63) / 64, t128 = (long long)((a.M + 127) / 128) * n64 * a.splits;
   if (a.N <= 32) return kT64x32;
-  return kT64;
+  if (t128 >= 256) return kT128x64;
+  return (long long)((a.M + 63) / 64) * n64 * a.splits >= 256 ? kT64x64 : kT64x32;
 }
 
-// Whole 64x64 tiles, every K slice (the last included) a multiple of 32,
-// 16-byte aligned rows and pointers for the DMA and the float4 epilogue, and
-// operands addressable with 32-bit byte offsets.
+// The split tiles address a stage by 32-bit byte offsets: at most 128 rows or
+// 64 k of either operand.  Longer rows go to the f32 MFMA tile.
+bool split_ok(const F32Args& a) { return a.lda <= (1 << 21) && a.ldb <= (1 << 21); }
+
+// Products that stay on the f32 MFMA tile: whole 64x64 tiles, every K slice
+// (the last included) a multiple of 32 and at most 512 long, too few tiles for
+// larger ones, 16-byte aligned rows and pointers, and operands addressable
+// with 32-bit byte offsets.  Over so short a K the split tile's longer
+// prologue costs what its matrix rate gains: 2048x1024, K 512 takes 20.6 us
+// here and 20.3 split (K 1024: 36.4 and 32.5), the batch-32 step's update
+// launch (K 32) 11.6 and 12.4.
 template <bool A_KC, bool B_KC>
-bool dma_ok(const F32Args& a) {
+bool dma_better(const F32Args& a) {
   const int last = a.K - (a.splits - 1) * a.k_per_split;
-  auto al = [](const void* ptr) { return (reinterpret_cast<uintptr_t>(ptr) & 15) == 0; };
-  const long long lim = 1LL << 31;
-  const bool epi_ok = (a.epi != RT_EPI_BIAS && a.epi != RT_EPI_BIAS_RELU) || al(a.bias);
-  const bool mask_ok = a.epi != RT_EPI_RELU_MASK || al(a.mask);
-  return a.M % 64 == 0 && a.N % 64 == 0 && a.k_per_split % 32 == 0 && last > 0 && last % 32 == 0 && a.vec_a &&
-         a.vec_b && a.vec_c && epi_ok && mask_ok && (long long)(A_KC ? a.M : a.K) * a.lda * 4 < lim &&
-         (long long)(B_KC ? a.N : a.K) * a.ldb * 4 < lim;
+  const long long lim = 1LL << 31, t128 = (long long)((a.M + 127) / 128) * ((a.N + 127) / 128) * a.splits;
+  return a.M % 64 == 0 && a.N % 64 == 0 && a.k_per_split <= 512 && a.k_per_split % 32 == 0 && last > 0 &&
+         last % 32 == 0 && t128 < 512 && a.vec_a && a.vec_b && a.vec_c &&
+         (long long)(A_KC ? a.M : a.K) * a.lda * 4 < lim && (long long)(B_KC ? a.N : a.K) * a.ldb * 4 < lim;
 }
 
-template <bool A_KC, bool B_KC>
-hipError_t launch_dma(hipStream_t s, F32Args a) {
-  using T = F32DmaTile<A_KC, B_KC>;
-  a.tiles_m = a.M / 64;
-  a.tiles_n = a.N / 64;
+// TN products (weight gradients) over at most 128 rows that dma_better leaves
+// out stay on the plain f32 tile, whose column sums are added row by row: the
+// bias gradient of a small batch then has the bits of the reference's
+// left-to-right sum.
+bool row_order_tn(const F32Args& a) { return a.splits <= 1 && a.K <= 128 && !dma_better<false, false>(a); }
+
+template <class T>
+hipError_t launch_tile(hipStream_t s, F32Args a) {
+  a.tiles_m = (a.M + T::BM - 1) / T::BM;
+  a.tiles_n = (a.N + T::BN - 1) / T::BN;
   dim3 grid(a.tiles_m * a.tiles_n, 1, a.splits);
   rt::launch((gemm_f32_kernel<T>), grid, dim3(T::THREADS), 0, s, a);
   return hipGetLastError();
@@ -1123,12 +1450,12 @@ hipError_t dispatch_tile(hipStream_t s, F32Args a) {
   if constexpr (A_KC && B_KC) {
     if (rank_k_ok(a)) return launch_rank_k(s, a);
   }
+  if (dma_better<A_KC, B_KC>(a)) return launch_tile<F32DmaTile<A_KC, B_KC>>(s, a);
+  if (!split_ok(a) || (!A_KC && row_order_tn(a))) return launch_tile<F32Tile<A_KC, B_KC>>(s, a);
   switch (pick_tile(a)) {
-    case kT128: return launch_f32<128, 128, A_KC, B_KC>(s, a);
-    case kT64x32: return launch_f32<64, 32, A_KC, B_KC>(s, a);
-    default:
-      if (dma_ok<A_KC, B_KC>(a)) return launch_dma<A_KC, B_KC>(s, a);
-      return launch_f32<64, 64, A_KC, B_KC>(s, a);
+    case kT128x64: return launch_tile<F32Split<2, 4, A_KC, B_KC>>(s, a);
+    case kT64x64: return launch_tile<F32Split<1, 4, A_KC, B_KC>>(s, a);
+    default: return launch_tile<F32Split<1, 2, A_KC, B_KC>>(s, a);
   }
 }
 
@@ -1156,19 +1483,19 @@ F32Args make_args(const rt::GemmDesc& d) {
   auto al16 = [](const void* ptr) { return (reinterpret_cast<uintptr_t>(ptr) & 15) == 0; };
   a.vec_a = (d.lda % 4 == 0) && al16(d.A);
   a.vec_b = (d.ldb % 4 == 0) && al16(d.B);
-  a.vec_c = (d.ldc % 4 == 0) && al16(d.C);
+  a.vec_c = (d.ldc % 4 == 0) && al16(d.C) && (d.bias == nullptr || al16(d.bias)) &&
+            (d.epi != RT_EPI_RELU_MASK || al16(d.mask)) && (d.splits <= 1 || d.split_stride % 4 == 0);
   return a;
 }
 
-// The backward pair of a hidden layer: dW = Aᵀ·δ (TN, 64x64 or, for a
-// narrow layer, 64x32 tiles; any number of K slices) and
-// dX = (δ·Wᵀ) ⊙ mask (NT, 64x64 tiles, whole K).
-template <class T0, class T1, int BN0>
+// The backward pair of a hidden layer: dW = Aᵀ·δ (TN, any number of K
+// slices) and dX = (δ·Wᵀ) ⊙ mask (NT, whole K).
+template <class T0, class T1>
 hipError_t launch_pair_tn_nt(hipStream_t s, F32Args a0, F32Args a1) {
-  a0.tiles_m = (a0.M + 63) / 64;
-  a0.tiles_n = (a0.N + BN0 - 1) / BN0;
-  a1.tiles_m = (a1.M + 63) / 64;
-  a1.tiles_n = (a1.N + 63) / 64;
+  a0.tiles_m = (a0.M + T0::BM - 1) / T0::BM;
+  a0.tiles_n = (a0.N + T0::BN - 1) / T0::BN;
+  a1.tiles_m = (a1.M + T1::BM - 1) / T1::BM;
+  a1.tiles_n = (a1.N + T1::BN - 1) / T1::BN;
   const long long nb0 = (long long)a0.tiles_m * a0.tiles_n * a0.splits;
   const long long nb1 = (long long)a1.tiles_m * a1.tiles_n * a1.splits;
   const long long n0 = (nb0 + 7) / 8 * 8;
@@ -1176,6 +1503,24 @@ hipError_t launch_pair_tn_nt(hipStream_t s, F32Args a0, F32Args a1) {
   rt::launch((gemm_f32_pair_kernel<T0, T1>), dim3((unsigned)(n0 + nb1)), dim3(T0::THREADS), 0, s, a0,
                      a1, (int)n0);
   return hipGetLastError();
+}
+
+// f(tile) for the dW of an update launch: the tile of its own launch.
+template <class F>
+hipError_t by_tn_tile(const F32Args& a, F&& f) {
+  if (dma_better<false, false>(a)) return f(F32DmaTile<false, false>{});
+  if (row_order_tn(a)) return f(F32Tile<false, false>{});
+  switch (pick_tile(a)) {
+    case kT128x64: return f(F32Split<2, 4, false, false>{});
+    case kT64x64: return f(F32Split<1, 4, false, false>{});
+    default: return f(F32Split<1, 2, false, false>{});
+  }
+}
+
+// f(64x64 tile) for a dW whose tiles update their layer.
+template <class F>
+hipError_t by_update_tile(const F32Args& a, F&& f) {  // whole 64x64 tiles (gemm_opt_update_ok)
+  return dma_better<false, false>(a) ? f(F32DmaTile<false, false>{}) : f(F32Split<1, 4, false, false>{});
 }
 
 }  // namespace
@@ -1196,10 +1541,10 @@ hipError_t gemm_f32_launch(hipStream_t s, const GemmDesc& d) {
   return hipErrorInvalidValue;
 }
 
-template <class T, int BM, int BN>
+template <class T>
 hipError_t launch_gemm_opt(hipStream_t s, F32Args a, const rt_opt::OptBatch& b, long long opt_blocks) {
-  a.tiles_m = (a.M + BM - 1) / BM;
-  a.tiles_n = (a.N + BN - 1) / BN;
+  a.tiles_m = (a.M + T::BM - 1) / T::BM;
+  a.tiles_n = (a.N + T::BN - 1) / T::BN;
   const long long n_gemm = (long long)a.tiles_m * a.tiles_n * a.splits;
   if (n_gemm + opt_blocks > 0x7fffffffLL) return hipErrorInvalidValue;
   rt::launch((gemm_f32_opt_kernel<T>), dim3((unsigned)(n_gemm + opt_blocks)), dim3(T::THREADS), 0, s, a, b,
@@ -1209,16 +1554,19 @@ hipError_t launch_gemm_opt(hipStream_t s, F32Args a, const rt_opt::OptBatch& b, 
 
 bool gemm_opt_supported(const GemmDesc& d, const OptTensor* ts, int nt, const OptParams& P) {
   if (d.in_dtype != RT_F32 || d.layout != RT_TN || d.M <= 0 || d.N <= 0 || d.K <= 0) return false;
-  return nt > 0 && optimizer_fits_cache(ts, nt, P);
+  return nt > 0 && (split_ok(make_args(d)) || row_order_tn(make_args(d))) && optimizer_fits_cache(ts, nt, P);
 }
 
 bool gemm_opt_update_ok(const GemmDesc& d, const OptTensor* wb, const OptParams& P) {
   if (d.in_dtype != RT_F32 || d.layout != RT_TN || d.splits > 1 || d.epi != RT_EPI_NONE || d.colsum == nullptr ||
       d.ldc != d.N || d.M <= 0 || d.N <= 0 || d.K <= 0)
     return false;
-  // The tile the TN GEMM's own launch would take: 64x64 DMA tiles.
+  // Whole 64x64 tiles with float4 stores; a product of 512 128x128 tiles or
+  // more is left to its own, larger tiles (and its update to the optimizer).
   const F32Args a = make_args(d);
-  if (pick_tile(a) != kT64 || !dma_ok<false, false>(a)) return false;
+  if (a.M % 64 != 0 || a.N % 64 != 0 || !a.vec_c || !split_ok(a) || row_order_tn(a) ||
+      (long long)((a.M + 127) / 128) * ((a.N + 127) / 128) >= 512)
+    return false;
   auto al16 = [](const void* ptr) { return (reinterpret_cast<uintptr_t>(ptr) & 15) == 0; };
   const OptTensor &W = wb[0], &Bt = wb[1];
   const bool adam = P.kind == 0, need_m = adam || P.momentum != 0.0f;
@@ -1248,17 +1596,14 @@ hipError_t gemm_opt_launch(hipStream_t s, const GemmDesc& d, const OptTensor* ts
     if (n_gemm + opt_blocks > 0x7fffffffLL) return hipErrorInvalidValue;
     UpdEpi u{upd[0], upd[1], P};
     u.P.skip_count = nullptr;  // counted by the optimizer blocks of the launch
-    rt::launch(gemm_f32_opt_upd_kernel, dim3((unsigned)(n_gemm + opt_blocks)), dim3(F32Dma::THREADS), 0, s, a, b,
-               (int)n_gemm, u);
-    return hipGetLastError();
+    return by_update_tile(a, [&](auto t) {
+      using T = decltype(t);
+      rt::launch(gemm_f32_opt_upd_kernel<T>, dim3((unsigned)(n_gemm + opt_blocks)), dim3(T::THREADS), 0, s, a, b,
+                 (int)n_gemm, u);
+      return hipGetLastError();
+    });
   }
-  switch (pick_tile(a)) {
-    case kT128: return launch_gemm_opt<F32Tile<128, 128, false, false>, 128, 128>(s, a, b, opt_blocks);
-    case kT64x32: return launch_gemm_opt<F32Tile<64, 32, false, false>, 64, 32>(s, a, b, opt_blocks);
-    default:
-      if (dma_ok<false, false>(a)) return launch_gemm_opt<F32DmaTile<false, false>, 64, 64>(s, a, b, opt_blocks);
-      return launch_gemm_opt<F32Tile<64, 64, false, false>, 64, 64>(s, a, b, opt_blocks);
-  }
+  return by_tn_tile(a, [&](auto t) { return launch_gemm_opt<decltype(t)>(s, a, b, opt_blocks); });
 }
 
 hipError_t gemm_opt_update2_launch(hipStream_t s, const GemmDesc& d0, const OptTensor* upd0, const GemmDesc& d1,
@@ -1280,33 +1625,39 @@ hipError_t gemm_opt_update2_launch(hipStream_t s, const GemmDesc& d0, const OptT
   if (n1 + opt_blocks > 0x7fffffffLL) return hipErrorInvalidValue;
   UpdEpi u0{upd0[0], upd0[1], P}, u1{upd1[0], upd1[1], P};
   u0.P.skip_count = u1.P.skip_count = nullptr;  // counted by the optimizer blocks of the launch
-  rt::launch(gemm_f32_opt_upd2_kernel, dim3((unsigned)(n1 + opt_blocks)), dim3(F32Dma::THREADS), 0, s, a0, a1, b,
-             (int)n0, (int)n1, u0, u1);
-  return hipGetLastError();
+  if (dma_better<false, false>(a0) != dma_better<false, false>(a1)) return hipErrorInvalidValue;  // one batch, one K
+  return by_update_tile(a0, [&](auto t) {
+    using T = decltype(t);
+    rt::launch(gemm_f32_opt_upd2_kernel<T>, dim3((unsigned)(n1 + opt_blocks)), dim3(T::THREADS), 0, s, a0, a1, b,
+               (int)n0, (int)n1, u0, u1);
+    return hipGetLastError();
+  });
 }
 
 bool gemm_pair_supported(const GemmDesc& d0, const GemmDesc& d1) {
   if (d0.in_dtype != RT_F32 || d1.in_dtype != RT_F32) return false;
   if (d0.layout != RT_TN || d1.layout != RT_NT || d1.splits > 1) return false;
-  // Only where the single launches would use the same tiles.
-  const TileCfg t0 = pick_tile(make_args(d0));
-  return (t0 == kT64 || t0 == kT64x32) && (pick_tile(make_args(d1)) == kT64 || rank_k_ok(make_args(d1)));
+  // Where the dW alone does not fill the chip with the largest tile.
+  const F32Args a0 = make_args(d0), a1 = make_args(d1);
+  return (split_ok(a0) || row_order_tn(a0)) && split_ok(a1) && pick_tile(a0) != kT128x64;
 }
 
 hipError_t gemm_pair_launch(hipStream_t s, const GemmDesc& d0, const GemmDesc& d1) {
   if (!gemm_pair_supported(d0, d1)) return hipErrorInvalidValue;
   const F32Args a0 = make_args(d0), a1 = make_args(d1);
-  // dX takes the block its single launch would (the rank-K block for K <= 16).
-  const bool rk = rank_k_ok(a1);
-  if (pick_tile(a0) == kT64x32)
-    return rk ? launch_pair_tn_nt<F32Tile<64, 32, false, false>, F32RankK, 32>(s, a0, a1)
-              : launch_pair_tn_nt<F32Tile<64, 32, false, false>, F32Tile<64, 64, true, true>, 32>(s, a0, a1);
-  if (rk)
-    return dma_ok<false, false>(a0) ? launch_pair_tn_nt<F32DmaTile<false, false>, F32RankK, 64>(s, a0, a1)
-                                    : launch_pair_tn_nt<F32Tile<64, 64, false, false>, F32RankK, 64>(s, a0, a1);
-  if (dma_ok<false, false>(a0) && dma_ok<true, true>(a1))
-    return launch_pair_tn_nt<F32DmaTile<false, false>, F32DmaTile<true, true>, 64>(s, a0, a1);
-  return launch_pair_tn_nt<F32Tile<64, 64, false, false>, F32Tile<64, 64, true, true>, 64>(s, a0, a1);
+  // dX takes the rank-K block for K <= 16, else the tile of its own launch;
+  // a dW next to it 64x64 tiles (the launch has blocks enough) unless it is
+  // narrow.  Each product is computed as in its own launch (same bits).
+  auto with_dx = [&](auto t0) {
+    using T0 = decltype(t0);
+    if (rank_k_ok(a1)) return launch_pair_tn_nt<T0, F32RankK>(s, a0, a1);
+    if (dma_better<true, true>(a1)) return launch_pair_tn_nt<T0, F32DmaTile<true, true>>(s, a0, a1);
+    return pick_tile(a1) == kT128x64 ? launch_pair_tn_nt<T0, F32Split<2, 4, true, true>>(s, a0, a1)
+                                     : launch_pair_tn_nt<T0, F32Split<1, 4, true, true>>(s, a0, a1);
+  };
+  if (dma_better<false, false>(a0)) return with_dx(F32DmaTile<false, false>{});
+  if (row_order_tn(a0)) return with_dx(F32Tile<false, false>{});
+  return a0.N <= 32 ? with_dx(F32Split<1, 2, false, false>{}) : with_dx(F32Split<1, 4, false, false>{});
 }
 
 hipError_t splitk_reduce_launch(hipStream_t s, const float* partials, int splits, long long stride, int M, int N,

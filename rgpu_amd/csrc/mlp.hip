@@ -336,7 +336,7 @@ static std::array<OptTensor, 2> layer_update(const rt_mlp* p, int l, const OptPa
   return {seg(Ly.w_off, Ly.din * Ly.dout), seg(Ly.b_off, Ly.dout)};
 }
 
-// Layer 0's dW of an f32 plan as one unsplit launch of DMA tiles: with the
+// Layer 0's dW of an f32 plan as one unsplit launch of 64x64 tiles: with the
 // update of layers 1.. in the same launch (fuse_update), its tiles also
 // update layer 0 itself (gemm_opt_update_ok), and the step has no optimizer
 // launch of its own.

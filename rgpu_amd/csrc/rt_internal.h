@@ -216,7 +216,8 @@ hipError_t gemm_launch(hipStream_t s, const GemmDesc& d);
 // float4-aligned: 16-column and 16-k blocks, K >= 128.
 bool gemm_f32_skinny_shape(int M, int N, int K);
 // Two independent GEMMs in one launch: d0 TN (any K slices) and d1 NT
-// (whole K), f32, where both would run on 64x64 tiles.  gemm_pair_supported
+// (whole K), f32, where the dW alone would not fill the chip with 128x64
+// tiles.  gemm_pair_supported
 // says whether gemm_pair_launch accepts the pair.
 bool gemm_pair_supported(const GemmDesc& d0, const GemmDesc& d1);
 hipError_t gemm_pair_launch(hipStream_t s, const GemmDesc& d0, const GemmDesc& d1);
