@@ -96,16 +96,20 @@ __device__ inline float half_to_f32(unsigned short h) {
 }
 
 // 8 consecutive halves of a row-major matrix at (row, col); zero outside.
-// One 16-byte load whenever the operand is 16-byte aligned (vec) and the whole
-// chunk is inside, so edge tiles stay vectorised except for their last chunk.
-__device__ inline u4 load8(const unsigned short* base, int ld, int row, int col, int rows, int cols, bool vec) {
+// One 16-byte load whenever the whole chunk is inside, whatever its alignment
+// (an odd row stride leaves it on 2 bytes; element by element such operands
+// 1500x777, K 1003 took 54.5 us, 26.2 this way), so edge tiles stay vectorised except for their last chunk.
+__device__ inline u4 load8(const unsigned short* base, int ld, int row, int col, int rows, int cols) {
   const unsigned short* src = base + (long long)row * ld + col;
-  if (vec && row < rows && col + 8 <= cols) return *reinterpret_cast<const u4*>(src);
+  u4 v;
+  if (row < rows && col + 8 <= cols) {
+    __builtin_memcpy(&v, src, 16);
+    return v;
+  }
   if (row >= rows) return u4{0u, 0u, 0u, 0u};
   unsigned short h[8];
 #pragma unroll
   for (int e = 0; e < 8; ++e) h[e] = (row < rows && col + e < cols) ? src[e] : (unsigned short)0;
-  u4 v;
 #pragma unroll
   for (int d = 0; d < 4; ++d) v[d] = (unsigned int)h[2 * d] | ((unsigned int)h[2 * d + 1] << 16);
   return v;
@@ -136,17 +140,16 @@ struct Operand {
   __device__ static inline int swz(int row, int granule) { return (granule ^ ((row >> 1) & 7)) * 8; }
 
   // Global (rows r0.., k0..) -> registers.
-  __device__ inline void load(const unsigned short* base, int ld, int r0, int k0, int rows, int ke, bool vec,
-                              int tid) {
+  __device__ inline void load(const unsigned short* base, int ld, int r0, int k0, int rows, int ke, int tid) {
 #pragma unroll
     for (int i = 0; i < PER_THREAD; ++i) {
       const int idx = tid + THREADS * i;
       if constexpr (KC) {
         const int row = idx / (BK / 8), kc = idx % (BK / 8);
-        v[i] = load8(base, ld, r0 + row, k0 + 8 * kc, rows, ke, vec);
+        v[i] = load8(base, ld, r0 + row, k0 + 8 * kc, rows, ke);
       } else {
         const int kk = idx / (ROWS / 8), c = idx % (ROWS / 8);
-        v[i] = load8(base, ld, k0 + kk, r0 + 8 * c, ke, rows, vec);
+        v[i] = load8(base, ld, k0 + kk, r0 + 8 * c, ke, rows);
       }
     }
   }
@@ -288,8 +291,8 @@ __global__ __launch_bounds__(64 * WGM * WGN) void gemm_half_kernel(HalfArgs p) {
   OpA oa;
   OpB ob;
   auto load_tiles = [&](int k0) {
-    oa.load(p.A, p.lda, m0, k0, p.M, ke, p.vec_a, tid);
-    ob.load(p.B, p.ldb, n0, k0, p.N, ke, p.vec_b, tid);
+    oa.load(p.A, p.lda, m0, k0, p.M, ke, tid);
+    ob.load(p.B, p.ldb, n0, k0, p.N, ke, tid);
   };
 
   f4 acc[TM][TN];
@@ -405,6 +408,7 @@ struct DmaOperand {
   // it for its first instruction (voff[1]: the odd instructions when PAR).
   __amdgpu_buffer_rsrc_t rsrc;
   int voff[2];
+  int vlast[2];   // edge tiles: the offsets for the last stage
   int row_bytes;  // bytes per stored row of the operand (2 ld)
 
   // K-contiguous: granule j of row r is stored at j ^ kc_sw(r).  16 lanes read
@@ -436,13 +440,37 @@ struct DmaOperand {
       }
     }
   }
+  // Edge tiles: the descriptor ends with the operand (`bytes` past the tile
+  // origin), so rows past the last one, and k rows past K, arrive as zeros.  A
+  // K-contiguous row's k past the last stage's `krem` would be the next row's
+  // first values: the lanes that hold them take an offset past the end.
+  __device__ inline void init_edge(const unsigned short* tile, int ld, int wave, int lane, long long bytes, int krem) {
+    init(tile, ld, wave, lane);
+    constexpr int END = 0x7ffffff0;
+    rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<unsigned short*>(tile), (short)0,
+                                             (int)(bytes < 0 ? 0LL : bytes < END ? bytes : (long long)END), 0x00020000);
+    bool past = false;
+    if constexpr (KC) {
+      const int row = (512 / BKD) * wave + lane / GR;
+      past = 8 * ((lane % GR) ^ kc_sw(row)) >= krem;
+    }
+#pragma unroll
+    for (int par = 0; par < 2; ++par) vlast[par] = past ? END : voff[par];
+  }
   // This wave's DMA of the stage `stage_bytes` past the tile origin into `lds`
   // (ASM: through rt_dev::dma16_asm, ordered only by the kernel's own waits).
-  template <bool ASM>
-  __device__ inline void issue(int stage_bytes, unsigned short* lds, int wave) const {
+  template <bool ASM, bool EDGE = false>
+  __device__ inline void issue(int stage_bytes, unsigned short* lds, int wave, bool last = false) const {
 #pragma unroll
     for (int i = 0; i < PER_WAVE; ++i) {
-      const int vo = voff[PAR ? (i & 1) : 0], so = stage_bytes + i * RSTEP * row_bytes;
+      const int par = PAR ? (i & 1) : 0;
+      int vo = voff[par], so = stage_bytes + i * RSTEP * row_bytes;
+      if constexpr (EDGE) {
+        // The whole offset in the vector part: the range check compares that
+        // with the descriptor's size (at most 2^32 - 1, so it cannot wrap).
+        vo = (last ? vlast[par] : vo) + so;
+        so = 0;
+      }
       if constexpr (ASM)
         rt_dev::dma16_asm(rsrc, lds + 512 * (i * WAVES + wave), vo, so);
       else
@@ -604,6 +632,76 @@ __device__ __forceinline__ void store_direct_any(const HalfArgs& p, const f4 (&a
   }
 }
 
+// store_direct for tiles that may reach past M or N, or whose rows do not
+// start on a vector store's alignment: the same lane layout, bounds checked.
+// Four columns go out as one store where they are inside and aligned.
+template <int TM, int TN>
+__device__ __forceinline__ void store_edge(const HalfArgs& p, const f4 (&acc)[TM][TN], int row0, int n0, int g, int r,
+                                           int slice) {
+  const bool partial = gridDim.z > 1, out_bf16 = !partial && p.out_bf16;
+  float* Cf = static_cast<float*>(p.C) + (partial ? (long long)slice * p.split_stride : 0);
+  unsigned short* Ch = static_cast<unsigned short*>(p.C);
+  const int epi = partial ? RT_EPI_NONE : p.epi;
+  const bool vec = p.ldc % 4 == 0 && (reinterpret_cast<uintptr_t>(out_bf16 ? (void*)Ch : (void*)Cf) & 15) == 0;
+  const bool vec_mask = p.ldc % 4 == 0 && (reinterpret_cast<uintptr_t>(p.mask) & 15) == 0;
+  static_for<0, TM>([&](auto tc) {
+    constexpr int t = decltype(tc)::value;
+    const int row = row0 + 16 * t + r;
+    if (row >= p.M) return;
+    const long long row_off = (long long)row * p.ldc;
+#pragma unroll
+    for (int u = 0; u < TN; ++u) {
+      const int col = n0 + 16 * u + 4 * g, nv = min(4, p.N - col);
+      if (nv <= 0) continue;
+      const long long off = row_off + col;
+      f4 v = acc[t][u];
+      if (epi == RT_EPI_BIAS || epi == RT_EPI_BIAS_RELU) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          if (e < nv) v[e] = v[e] + p.bias[col + e];
+          if (epi == RT_EPI_BIAS_RELU) v[e] = fmaxf(v[e], 0.0f);
+        }
+      } else if (epi == RT_EPI_RELU_MASK) {
+        f4 mk;
+        if (vec_mask && nv == 4 && p.mask_bf16) {
+          const u2 h = *reinterpret_cast<const u2*>(static_cast<const unsigned short*>(p.mask) + off);
+          mk = f4{__uint_as_float(h[0] << 16), __uint_as_float(h[0] & 0xffff0000u), __uint_as_float(h[1] << 16),
+                  __uint_as_float(h[1] & 0xffff0000u)};
+        } else if (vec_mask && nv == 4) {
+          mk = *reinterpret_cast<const f4*>(static_cast<const float*>(p.mask) + off);
+        } else {
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            mk[e] = e >= nv ? 0.0f
+                    : p.mask_bf16 ? bf16_to_f32(static_cast<const unsigned short*>(p.mask)[off + e])
+                                  : static_cast<const float*>(p.mask)[off + e];
+        }
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          if (!(mk[e] > 0.0f)) v[e] = 0.0f;
+      }
+      if (out_bf16) {
+        unsigned short h[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) h[e] = f32_to_bf16_rne(v[e]);
+        if (vec && nv == 4) {
+          *reinterpret_cast<u2*>(Ch + off) = u2{h[0] | ((unsigned)h[1] << 16), h[2] | ((unsigned)h[3] << 16)};
+        } else {
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            if (e < nv) Ch[off + e] = h[e];
+        }
+      } else if (vec && nv == 4) {
+        *reinterpret_cast<f4*>(Cf + off) = v;
+      } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          if (e < nv) Cf[off + e] = v[e];
+      }
+    }
+  });
+}
+
 // Two LDS stages of BKD = 64 k (two MFMA k-steps, kk = 0, 1).  With the
 // fragments of (stage k, kk 0) already in registers, stage k runs as
 //   A: read (k, kk 1) fragments       | MFMAs of (k, kk 0)
@@ -612,8 +710,13 @@ __device__ __forceinline__ void store_direct_any(const HalfArgs& p, const f4 (&a
 // so every LDS read overlaps MFMAs and there is one barrier per 64 k.  The
 // reads and the DMA are interleaved one per MFMA: a single wave per SIMD
 // never stalls on a full memory queue with MFMAs still to issue.
-template <int BM, int BN, int WGM, int WGN, bool A_KC, bool B_KC, bool IS_BF16, int BKD, int NS>
-__global__ __launch_bounds__(64 * WGM * WGN) void gemm_half_dma_kernel(HalfArgs p) {
+//
+// EDGE: tiles that may reach past M, N or K (rows a multiple of 8 halves).
+// The DMA then zero-fills what lies outside, and the stores check bounds: the
+// layer 4100 x 4000 -> 1000 forward and backward 428 us on the register-staged
+// kernel, 195 here.
+template <int BM, int BN, int WGM, int WGN, bool A_KC, bool B_KC, bool IS_BF16, int BKD, int NS, bool EDGE>
+__device__ __forceinline__ void dma_body(const HalfArgs& p) {
   constexpr int THREADS = 64 * WGM * WGN;
   constexpr int WM = BM / WGM, WN = BN / WGN;
   constexpr int TM = WM / 16, TN = WN / 16;
@@ -621,7 +724,8 @@ __global__ __launch_bounds__(64 * WGM * WGN) void gemm_half_dma_kernel(HalfArgs 
   using OpB = DmaOperand<BN, B_KC, THREADS, BKD>;
   constexpr int STAGE = OpA::ELEMS + OpB::ELEMS;
   constexpr int PER_STAGE = OpA::PER_WAVE + OpB::PER_WAVE;  // DMA instructions per wave per stage
-  static_assert(BKD == 64 && NS == 2, "two stages of two MFMA k-steps");
+  static_assert(BKD == 64 && NS >= 2, "stages of two MFMA k-steps");
+  static_assert((NS - 1) * PER_STAGE < 64, "vmcnt range");
   __shared__ __attribute__((aligned(16))) unsigned short smem[NS * STAGE];
   auto sA = [&](int buf) { return smem + buf * STAGE; };
   auto sB = [&](int buf) { return smem + buf * STAGE + OpA::ELEMS; };
@@ -657,12 +761,23 @@ __global__ __launch_bounds__(64 * WGM * WGN) void gemm_half_dma_kernel(HalfArgs 
   const int m0 = tile_m * BM, n0 = tile_n * BN;
 
   const int kb = slice * p.k_per_split;
-  const int nk = (min(p.K, kb + p.k_per_split) - kb) / BKD;  // whole stages (checked by the host)
+  const int kn = min(p.K, kb + p.k_per_split) - kb;
+  const int nk = EDGE ? (max(kn, 0) + BKD - 1) / BKD : kn / BKD;  // whole stages, checked by the host, unless EDGE
 
   OpA oa;
   OpB ob;
-  oa.init(A_KC ? p.A + (long long)m0 * p.lda + kb : p.A + (long long)kb * p.lda + m0, p.lda, wave, lane);
-  ob.init(B_KC ? p.B + (long long)n0 * p.ldb + kb : p.B + (long long)kb * p.ldb + n0, p.ldb, wave, lane);
+  const unsigned short* const a0 = A_KC ? p.A + (long long)m0 * p.lda + kb : p.A + (long long)kb * p.lda + m0;
+  const unsigned short* const b0 = B_KC ? p.B + (long long)n0 * p.ldb + kb : p.B + (long long)kb * p.ldb + n0;
+  if constexpr (EDGE) {
+    const int krem = kn - (nk - 1) * BKD;
+    const long long a_end = A_KC ? (long long)(p.M - m0) * p.lda - kb : (long long)(p.K - kb) * p.lda - m0;
+    const long long b_end = B_KC ? (long long)(p.N - n0) * p.ldb - kb : (long long)(p.K - kb) * p.ldb - n0;
+    oa.init_edge(a0, p.lda, wave, lane, 2 * a_end, krem);
+    ob.init_edge(b0, p.ldb, wave, lane, 2 * b_end, krem);
+  } else {
+    oa.init(a0, p.lda, wave, lane);
+    ob.init(b0, p.ldb, wave, lane);
+  }
   const int a_step = 2 * (A_KC ? BKD : BKD * p.lda);  // bytes per stage
   const int b_step = 2 * (B_KC ? BKD : BKD * p.ldb);
   // With an M/N-contiguous B the DMA goes through inline asm: the compiler's
@@ -670,10 +785,12 @@ __global__ __launch_bounds__(64 * WGM * WGN) void gemm_half_dma_kernel(HalfArgs 
   // fragment read of stage k, halving the time each stage has to arrive
   // (measured: 4096^3 NN 117 -> 105 us, the K = 262144 split-K dW 159 -> 143
   // us).  The NT kernel's schedule has no such wait and keeps the builtin.
-  constexpr bool ASM_DMA = !B_KC;
+  // A deeper ring must not wait for every load in flight, so it takes the asm
+  // form too.
+  constexpr bool ASM_DMA = !B_KC || NS > 2;
   auto issue = [&](int stage, int buf) {
-    oa.template issue<ASM_DMA>(stage * a_step, sA(buf), wave);
-    ob.template issue<ASM_DMA>(stage * b_step, sB(buf), wave);
+    oa.template issue<ASM_DMA, EDGE>(stage * a_step, sA(buf), wave, stage == nk - 1);
+    ob.template issue<ASM_DMA, EDGE>(stage * b_step, sB(buf), wave, stage == nk - 1);
   };
 
   f4 acc[TM][TN];
@@ -757,43 +874,43 @@ __global__ __launch_bounds__(64 * WGM * WGN) void gemm_half_dma_kernel(HalfArgs 
     // the last stage it re-fetches stage nk-1 into a buffer nothing reads),
     // so the bookkeeping is the same in every stage.
     issue(0, 0);
-    issue(min(1, nk - 1), 1);
-    wait_vm<PER_STAGE>();
+    static_for<1, NS>([&](auto ic) { issue(min((int)decltype(ic)::value, nk - 1), decltype(ic)::value); });
+    wait_vm<(NS - 1) * PER_STAGE>();
     barrier_lds();
     read_frags(0, 0, fa0, fb0);
     auto stage = [&](int k, auto bc) {
-      constexpr int BUF = decltype(bc)::value;  // k % 2
+      constexpr int BUF = decltype(bc)::value, NEXT = (BUF + 1) % NS;  // k % NS
       // A: (k, kk 1) fragments in, (k, kk 0) MFMAs.
       read_frags(BUF, 1, fa1, fb1);
       mfmas(fa0, fb0);
       interleave(std::integral_constant<int, 0>{});
       if (!cs_shared || k % p.tiles_m == tile_m) colsum(BUF);
       // B: stage k+1 everywhere; stage k no longer read.
-      wait_vm<0>();
+      wait_vm<(NS - 2) * PER_STAGE>();
       barrier_lds();
       // (k+1, kk 0) fragments (discarded after the last stage) and the DMA of
-      // stage k+2 touch different buffers.  The DMA has one stage of MFMAs
+      // stage k+NS touch different buffers.  The DMA has NS - 1 stages of MFMAs
       // to land, so it starts right after the barrier: NT issues all of it
       // first; with a transposed operand A's half goes first, then the
       // fragment reads, then B's half (measured fastest of the orders tried:
       // reads first, DMA first, and the B-first mirror).
-      const int next = min(k + 2, nk - 1);
+      const int next = min(k + NS, nk - 1);
       if constexpr (A_KC && B_KC) {
         issue(next, BUF);
-        read_frags(BUF ^ 1, 0, fa0, fb0);
+        read_frags(NEXT, 0, fa0, fb0);
       } else {
-        oa.template issue<ASM_DMA>(next * a_step, sA(BUF), wave);
-        read_frags(BUF ^ 1, 0, fa0, fb0);
-        ob.template issue<ASM_DMA>(next * b_step, sB(BUF), wave);
+        oa.template issue<ASM_DMA, EDGE>(next * a_step, sA(BUF), wave, next == nk - 1);
+        read_frags(NEXT, 0, fa0, fb0);
+        ob.template issue<ASM_DMA, EDGE>(next * b_step, sB(BUF), wave, next == nk - 1);
       }
       mfmas(fa1, fb1);
       interleave(std::integral_constant<int, PER_STAGE>{});
     };
-    using B0 = std::integral_constant<int, 0>;
-    using B1 = std::integral_constant<int, 1>;
-    for (int k = 0; k < nk; k += 2) {
-      stage(k, B0{});
-      if (k + 1 < nk) stage(k + 1, B1{});
+    for (int k = 0; k < nk; k += NS) {
+      stage(k, std::integral_constant<int, 0>{});
+      static_for<1, NS>([&](auto ic) {
+        if (k + decltype(ic)::value < nk) stage(k + decltype(ic)::value, ic);
+      });
     }
   }
   wait_vm<0>();     // no DMA (the re-fetches past the last stage) still writing LDS
@@ -817,7 +934,20 @@ __global__ __launch_bounds__(64 * WGM * WGN) void gemm_half_dma_kernel(HalfArgs 
     if (bad && p.nf_flag && !cs_shared) *p.nf_flag = 1;  // shares are checked once summed
   }
 
-  store_direct_any<TM, TN>(p, acc, m0, n0, wm, wn, g, r, slice);
+  if constexpr (EDGE)
+    store_edge<TM, TN>(p, acc, m0 + wm, n0 + wn, g, r, slice);
+  else
+    store_direct_any<TM, TN>(p, acc, m0, n0, wm, wn, g, r, slice);
+}
+
+template <int BM, int BN, int WGM, int WGN, bool A_KC, bool B_KC, bool IS_BF16, int BKD, int NS>
+__global__ __launch_bounds__(64 * WGM * WGN) void gemm_half_dma_kernel(HalfArgs p) {
+  dma_body<BM, BN, WGM, WGN, A_KC, B_KC, IS_BF16, BKD, NS, false>(p);
+}
+
+template <int BM, int BN, int WGM, int WGN, bool A_KC, bool B_KC, bool IS_BF16, int BKD, int NS>
+__global__ __launch_bounds__(64 * WGM * WGN) void gemm_half_edge_kernel(HalfArgs p) {
+  dma_body<BM, BN, WGM, WGN, A_KC, B_KC, IS_BF16, BKD, NS, true>(p);
 }
 
 // dst[z, n] = sum over t of parts[z * rows + t, n], t in increasing order:
@@ -842,8 +972,13 @@ __global__ __launch_bounds__(256) void cs_shares_reduce_kernel(const float* __re
   if (nf_flag && not_finite(v)) *nf_flag = 1;
 }
 
-// Direct-to-LDS pipeline shape: K per stage and number of stages.
-constexpr int kDmaBK = 64, kDmaStages = 2;
+// Direct-to-LDS pipeline shape: K per stage and number of stages.  A CU needs
+// about 128 KB of loads on their way to keep its matrix cores fed (a stage
+// takes ~2000 cycles to arrive): one 256x256 block or two 128x128 blocks hold
+// that in two stages; where a smaller tile has its CU almost to itself, the
+// deep ring holds four (4000x1000, K 4100 TN on 256 128x128 blocks: 55.5 us in
+// two stages, 45.1 in four).
+constexpr int kDmaBK = 64, kDmaStages = 2, kDeepStages = 4;
 
 template <int BM, int BN>
 void set_tiles(HalfArgs& a) {
@@ -873,8 +1008,8 @@ bool dma_addressable(const HalfArgs& a) {
   return (long long)(A_KC ? a.M : a.K) * a.lda * 2 < lim && (long long)(B_KC ? a.N : a.K) * a.ldb * 2 < lim;
 }
 
-template <int BM, int BN, int WGM, int WGN, bool A_KC, bool B_KC>
-hipError_t launch_dma(hipStream_t s, HalfArgs a, int splits, bool bf16, float* cs_scratch = nullptr,
+template <int BM, int BN, int WGM, int WGN, bool A_KC, bool B_KC, int NS>
+hipError_t launch_dma(hipStream_t s, HalfArgs a, int splits, bool bf16, bool edge, float* cs_scratch = nullptr,
                       size_t cs_scratch_elems = 0, bool shares_to_caller = false) {
   set_tiles<BM, BN>(a);
   // Column sums shared over the M tiles when there are several and room.
@@ -883,12 +1018,13 @@ hipError_t launch_dma(hipStream_t s, HalfArgs a, int splits, bool bf16, float* c
       (size_t)splits * a.tiles_m * a.N <= cs_scratch_elems)
     a.cs_parts = cs_scratch;
   const dim3 grid(a.tiles_m * a.tiles_n, 1, splits), block(64 * WGM * WGN);
-  if (bf16)
-    rt::launch((gemm_half_dma_kernel<BM, BN, WGM, WGN, A_KC, B_KC, true, kDmaBK, kDmaStages>), grid, block, 0,
-                       s, a);
+  auto go = [&](auto kernel) { rt::launch(kernel, grid, block, 0, s, a); };
+  if (edge)
+    bf16 ? go(gemm_half_edge_kernel<BM, BN, WGM, WGN, A_KC, B_KC, true, kDmaBK, NS>)
+         : go(gemm_half_edge_kernel<BM, BN, WGM, WGN, A_KC, B_KC, false, kDmaBK, NS>);
   else
-    rt::launch((gemm_half_dma_kernel<BM, BN, WGM, WGN, A_KC, B_KC, false, kDmaBK, kDmaStages>), grid, block,
-                       0, s, a);
+    bf16 ? go(gemm_half_dma_kernel<BM, BN, WGM, WGN, A_KC, B_KC, true, kDmaBK, NS>)
+         : go(gemm_half_dma_kernel<BM, BN, WGM, WGN, A_KC, B_KC, false, kDmaBK, NS>);
   if (a.cs_parts && !shares_to_caller) {
     const long long n = (long long)splits * a.N;
     rt::launch(cs_shares_reduce_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, a.cs_parts,
@@ -910,20 +1046,34 @@ hipError_t launch_regs(hipStream_t s, HalfArgs a, int splits, bool bf16) {
 
 // Tile size (256, 128 or 64) and kernel (direct-to-LDS or register-staged)
 // for a problem: 256x256 blocks when they give at least one block per CU,
-// 128x128 for mid sizes, 64x64 for small ones.  Full tiles take the
-// direct-to-LDS kernel (256x256: two waves per SIMD with 128x64 wave tiles);
-// the rest the register-staged kernel.
+// 128x128 for mid sizes, 64x64 for small ones.  Whole tiles take the
+// direct-to-LDS kernel (256x256: two waves per SIMD with 128x64 wave tiles),
+// other sizes its form with bounds; the register-staged kernel is left with
+// rows that are no multiple of 8 halves (the DMA moves 16 aligned bytes).
 struct HalfPath {
   int tile;
-  bool dma;
+  bool dma;   // whole tiles
+  bool edge;  // direct-to-LDS loads too, but tiles may reach past the edges
+  bool deep;  // ... through kDeepStages LDS stages
 };
 template <bool A_KC, bool B_KC>
 HalfPath pick_path(const HalfArgs& a, int splits, bool overread_ok) {
   const long long tbig = (long long)((a.M + 255) / 256) * ((a.N + 255) / 256) * splits;
   const long long t128 = (long long)((a.M + 127) / 128) * ((a.N + 127) / 128) * splits;
-  const int tile = tbig >= 256 ? 256 : t128 >= 128 ? 128 : 64;
+  // A 256x256 block has its CU to itself, so a last round of few blocks costs
+  // a whole one (4100x4000, K 1000: 272 blocks 94.5 us, as 1056 128x128
+  // blocks 83.8).
+  const bool idle_round = (tbig + 255) / 256 * 256 > tbig * 4 / 3;
+  const int tile = tbig >= 256 && !idle_round ? 256 : t128 >= 128 ? 128 : 64;
+  // Four stages leave room for one 128x128 block per CU.
+  const bool deep = tile == 64 || (tile == 128 && t128 <= 256);
   // A ragged N is read past its end only along B's rows (N-contiguous B).
-  return HalfPath{tile, full_tiles(a, splits, tile, tile, overread_ok && !B_KC) && dma_addressable<A_KC, B_KC>(a)};
+  const bool addressable = dma_addressable<A_KC, B_KC>(a);
+  const bool dma = full_tiles(a, splits, tile, tile, overread_ok && !B_KC) && addressable;
+  // Slices (all but the last) are whole stages, so only the last can be cut by
+  // K; every element of a K-contiguous row lies in a whole 8-half chunk.
+  const bool short_rows = a.lda <= (1 << 21) && a.ldb <= (1 << 21);  // offsets of a whole tile or stage below 2^31
+  return HalfPath{tile, dma, !dma && addressable && short_rows && a.vec_a && a.vec_b && a.K > 0, deep};
 }
 
 template <bool A_KC, bool B_KC>
@@ -938,18 +1088,22 @@ hipError_t launch_half(hipStream_t s, HalfArgs a, int splits, bool bf16, float* 
       (!hp.dma || splits > 1 || a.n_ragged || a.M % 16 != 0 || a.N % 64 != 0 ||
        (a.relu_bits_out && !(a.epi == RT_EPI_BIAS_RELU && a.out_bf16)) || (a.relu_bits && a.epi != RT_EPI_RELU_MASK)))
     return hipErrorInvalidValue;
+  const bool direct = hp.dma || hp.edge;
   switch (hp.tile) {
     case 256:
-      return hp.dma ? launch_dma<256, 256, 2, 4, A_KC, B_KC>(s, a, splits, bf16, cs_scratch, cs_elems,
-                                                             shares_to_caller)
+      return direct ? launch_dma<256, 256, 2, 4, A_KC, B_KC, kDmaStages>(s, a, splits, bf16, hp.edge, cs_scratch,
+                                                                         cs_elems, shares_to_caller)
                     : launch_regs<256, 256, 4, 2, A_KC, B_KC>(s, a, splits, bf16);
     case 128:
-      return hp.dma ? launch_dma<128, 128, 2, 2, A_KC, B_KC>(s, a, splits, bf16, cs_scratch, cs_elems,
-                                                             shares_to_caller)
+      if (direct && hp.deep)
+        return launch_dma<128, 128, 2, 2, A_KC, B_KC, kDeepStages>(s, a, splits, bf16, hp.edge, cs_scratch, cs_elems,
+                                                                   shares_to_caller);
+      return direct ? launch_dma<128, 128, 2, 2, A_KC, B_KC, kDmaStages>(s, a, splits, bf16, hp.edge, cs_scratch,
+                                                                         cs_elems, shares_to_caller)
                     : launch_regs<128, 128, 2, 2, A_KC, B_KC>(s, a, splits, bf16);
     default:
-      return hp.dma ? launch_dma<64, 64, 2, 2, A_KC, B_KC>(s, a, splits, bf16, cs_scratch, cs_elems,
-                                                           shares_to_caller)
+      return direct ? launch_dma<64, 64, 2, 2, A_KC, B_KC, kDeepStages>(s, a, splits, bf16, hp.edge, cs_scratch,
+                                                                        cs_elems, shares_to_caller)
                     : launch_regs<64, 64, 2, 2, A_KC, B_KC>(s, a, splits, bf16);
   }
 }
@@ -960,7 +1114,7 @@ template <bool A_KC, bool B_KC>
 int half_share_rows(const HalfArgs& a, int splits, size_t cs_elems, bool have_scratch, bool overread_ok) {
   if (B_KC || !a.colsum || !have_scratch) return 0;
   const HalfPath hp = pick_path<A_KC, B_KC>(a, splits, overread_ok);
-  if (!hp.dma) return 0;
+  if (!hp.dma && !hp.edge) return 0;
   const int tiles_m = (a.M + hp.tile - 1) / hp.tile;
   return (tiles_m > 1 && (size_t)splits * tiles_m * a.N <= cs_elems) ? tiles_m : 0;
 }

@@ -1,0 +1,89 @@
+"""bf16 / f16 products whose sizes are no multiples of a tile: the
+direct-to-LDS kernel with bounds (rows a multiple of 8), and unaligned rows,
+against float64 on the rounded operands."""
+import numpy as np
+import pytest
+
+import rgpu_amd.gpu as G
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def gpu():
+    return G.Gpu(0)
+
+
+def rounded(a, dt):
+    return G.bf16_bits_to_f32(G.f32_to_bf16_bits(a)) if dt == G.BF16 else a.astype(np.float16).astype(np.float32)
+
+
+# K, M and N around the 64-k stage and the 64, 128 and 256 tiles; the last
+# three have odd rows (the register-staged kernel).
+SHAPES = [(8, 8, 8), (65, 72, 56), (66, 64, 72), (129, 136, 200), (1000, 1032, 64), (1500, 2040, 136), (264, 2000, 328),
+          (4100, 4104, 72), (4100, 1000, 520), (63, 65, 67), (130, 1001, 77), (300, 255, 1003)]
+
+
+@pytest.mark.parametrize("layout", [G.NN, G.TN, G.NT])
+@pytest.mark.parametrize("m,n,k", SHAPES)
+@pytest.mark.parametrize("dt", [G.BF16, G.F16])
+def test_product_bias_mask_and_colsum(gpu, layout, m, n, k, dt):
+    rng = np.random.default_rng(m + 3 * n + 7 * k)
+    a, b = (rounded(rng.standard_normal(s).astype(np.float32), dt) for s in ((m, k), (k, n)))
+    da = np.ascontiguousarray(a.T if layout == G.TN else a)
+    db = np.ascontiguousarray(b.T if layout == G.NT else b)
+    a64, b64 = a.astype(np.float64), b.astype(np.float64)
+    exact, mag = a64 @ b64, np.abs(a64) @ np.abs(b64)
+    # the products are exact; one rounding of the running sum per MFMA
+    tol = ((k + 31) // 32 + 4) * 2.0 ** -23 * mag
+    A, B, c = gpu.upload(da, dt), gpu.upload(db, dt), gpu.empty((m, n))
+    cs = gpu.empty((1, n)) if layout == G.TN else None
+    gpu.gemm(layout, A, B, c, colsum=cs)
+    assert np.all(np.abs(gpu.download(c) - exact) <= tol)
+    if cs is not None:
+        assert np.all(np.abs(gpu.download(cs)[0] - b64.sum(0)) <= k * 2.0 ** -24 * np.abs(b64).sum(0) + 1e-30)
+    bias = rng.standard_normal((1, n)).astype(np.float32)
+    gpu.gemm(layout, A, B, c, G.EPI_BIAS_RELU, gpu.upload(bias))
+    assert np.all(np.abs(gpu.download(c) - np.maximum(exact + bias, 0)) <= tol + 2.0 ** -23 * np.abs(bias))
+    if dt == G.BF16:  # bf16 results, masked
+        h = gpu.empty((m, n), G.BF16)
+        mask = rounded(rng.standard_normal((m, n)).astype(np.float32), dt)
+        gpu.gemm(layout, A, B, h, G.EPI_RELU_MASK, gpu.upload(mask, G.BF16))
+        got = gpu.download_f32(h)
+        assert np.all(np.abs(got - exact * (mask > 0)) <= tol + 2.0 ** -8 * np.abs(exact))
+
+
+@pytest.mark.parametrize("layout", [G.NN, G.TN, G.NT])
+def test_what_lies_past_an_edge_does_not_reach_the_result(gpu, layout):
+    """A row of infinities next to another row's K remainder, and operands
+    that end where their buffer ends."""
+    m, n, k = 136, 72, 72
+    rng = np.random.default_rng(3)
+    a, b = (rounded(rng.standard_normal(s).astype(np.float32), G.BF16) for s in ((m, k), (k, n)))
+    a[50, :] = np.inf
+    b[:, 20] = np.inf
+    da = np.ascontiguousarray(a.T if layout == G.TN else a)
+    db = np.ascontiguousarray(b.T if layout == G.NT else b)
+    c = gpu.empty((m, n))
+    gpu.gemm(layout, gpu.upload(da, G.BF16), gpu.upload(db, G.BF16), c)
+    got = gpu.download(c)
+    keep = np.ix_([i for i in range(m) if i != 50], [j for j in range(n) if j != 20])
+    a0, b0 = a.copy(), b.copy()
+    a0[50], b0[:, 20] = 0, 0
+    exact, mag = a0.astype(np.float64) @ b0, np.abs(a0).astype(np.float64) @ np.abs(b0)
+    assert np.all(np.abs(got - exact)[keep] <= 8 * 2.0 ** -23 * mag[keep])
+    assert not np.isfinite(got[50]).any() and not np.isfinite(got[:, 20]).any()
+
+
+@pytest.mark.parametrize("dt", [G.BF16, G.F16])
+@pytest.mark.parametrize("m,n,k,slices", [(72, 136, 1000, 4), (520, 264, 5000, 16), (72, 72, 200, 8), (130, 77, 3001, 8)])
+def test_slices(gpu, dt, m, n, k, slices):
+    """K slices of a ragged product: the last slice cut, or empty."""
+    rng = np.random.default_rng(k)
+    a, b = (rounded(rng.standard_normal(s).astype(np.float32), dt) for s in ((k, m), (k, n)))
+    dw, cs = gpu.empty((m, n)), gpu.empty((1, n))
+    gpu.split_k(gpu.upload(a, dt), gpu.upload(b, dt), dw, gpu.empty((slices * (m * n + n),)), slices, True, colsum=cs)
+    a64, b64 = a.astype(np.float64), b.astype(np.float64)
+    tol = ((k + 31) // 32 + slices + 4) * 2.0 ** -23 * (np.abs(a64).T @ np.abs(b64))
+    assert np.all(np.abs(gpu.download(dw) - a64.T @ b64) <= tol)
+    assert np.all(np.abs(gpu.download(cs)[0] - b64.sum(0)) <= k * 2.0 ** -24 * np.abs(b64).sum(0))
