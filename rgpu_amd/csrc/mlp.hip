@@ -648,7 +648,7 @@ int rt_mlp_create(rt_ctx* c, int n_layers, const size_t* dims, const float* cons
   n += opt_launches(p);  // optimizer
   if (p->mixed) {
     n += 1;  // step prologue
-    int unchecked = 0;  // layers whose dW GEMM cannot flag non-finite values itself
+    int unchecked = 0;  // tensors of the layers whose dW GEMM cannot flag non-finite values itself
     int jobs = 0;       // whole dW launches whose db shares the check launch adds
     for (int l = 0; l < n_layers; ++l) {
       const Layer& Ly = p->L[l];
@@ -657,11 +657,12 @@ int rt_mlp_create(rt_ctx* c, int n_layers, const size_t* dims, const float* cons
                               nullptr, nullptr, RT_F32, p->grad + Ly.b_off, Ly.splits_dw);
       layer_shares(Ly, dw);
       dw.nf_flag = p->state + 1;
-      unchecked += !gemm_checks_nonfinite(dw);
-      jobs += Ly.splits_dw <= 1 && gemm_cs_share_rows(dw) > 0;
+      const bool job = Ly.splits_dw <= 1 && gemm_cs_share_rows(dw) > 0;
+      if (!gemm_checks_nonfinite(dw)) unchecked += job ? 1 : 2;  // a share job checks its db itself
+      jobs += job;
     }
     // Separate checks, 24 tensors and 32 share jobs per launch.
-    n += std::max((jobs + kMaxShareJobs - 1) / kMaxShareJobs, (2 * unchecked + kMaxOptTensors - 1) / kMaxOptTensors);
+    n += std::max((jobs + kMaxShareJobs - 1) / kMaxShareJobs, (unchecked + kMaxOptTensors - 1) / kMaxOptTensors);
   }
   p->dispatches = n;
   c->mlps.push_back(p);
@@ -734,7 +735,7 @@ int rt_mlp_step(rt_mlp* p, const rt_buf* x, const rt_buf* labels) {
   const bool fold = fold_l1(p, x->ptr);  // layer 1's dW (and update) in that launch too
 
   const int in_dtype = p->mixed ? RT_BF16 : RT_F32;
-  std::vector<char> unchecked(nl, 1);
+  std::vector<char> unchecked(nl, 1), job(nl, 0);
   std::vector<ShareJob> jobs;
   for (int l = nl - 1; l >= 0; --l) {
     Layer& Ly = p->L[l];
@@ -755,6 +756,7 @@ int rt_mlp_step(rt_mlp* p, const rt_buf* x, const rt_buf* labels) {
       if (unchecked[l]) dw.nf_flag = nullptr;
       const int rows = dw.splits <= 1 ? gemm_cs_share_rows(dw) : 0;
       if (rows > 0) jobs.push_back(ShareJob{Ly.cs_shares, p->grad + Ly.b_off, rows, (int)Ly.dout});
+      job[l] = rows > 0;
     }
     if (l == 0) {
       const std::vector<OptTensor> rest = fuse ? plan_tensors(p, fold ? 2 : 1, nl, P) : std::vector<OptTensor>();
@@ -829,6 +831,7 @@ int rt_mlp_step(rt_mlp* p, const rt_buf* x, const rt_buf* labels) {
       if (!unchecked[l]) continue;
       ptrs.push_back(p->grad + p->L[l].w_off);
       ns.push_back(p->L[l].din * p->L[l].dout);
+      if (job[l]) continue;  // this launch writes that db, and checks it as it does
       ptrs.push_back(p->grad + p->L[l].b_off);
       ns.push_back(p->L[l].dout);
     }
