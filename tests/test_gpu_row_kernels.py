@@ -88,3 +88,18 @@ def test_rows_that_are_not_finite(gpu):
     assert np.isnan(got[0]).all() and np.isnan(got[2]).all() and np.isnan(got[1, 3])
     assert got[3, 5] == 0.0 and np.isclose(got[3, 0], 1 / 69)
     assert np.allclose(got[4:], 1 / 70)
+
+
+# Rows at the edges of the column kernel's stages (256) and add batches (32),
+# below its range too; columns at the edges of its blocks (16).
+@pytest.mark.parametrize("cols", [2, 15, 16, 17, 1000])
+@pytest.mark.parametrize("rows", [2, 31, 32, 33, 255, 256, 257, 512, 2083])
+def test_reduce_to_columns(gpu, rows, cols):
+    x = np.random.default_rng(rows * 10007 + cols).standard_normal((rows, cols)).astype(np.float32)
+    x[:, 0] = -0.0  # 0 + -0 stays +0
+    x[rows // 2, 1] = np.inf
+    out = gpu.empty((1, cols))
+    gpu.reduce_to(gpu.upload(x), out)
+    # added one by one in row order (tensor.rs:399-438): the same bits
+    want = np.add.accumulate(np.concatenate([np.zeros((1, cols), np.float32), x]), axis=0, dtype=np.float32)[-1:]
+    assert np.array_equal(gpu.download(out).view(np.uint32), want.view(np.uint32))
