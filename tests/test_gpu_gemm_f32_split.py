@@ -135,3 +135,15 @@ def test_small_magnitudes_keep_their_precision(gpu):
     gpu.gemm(G.NN, gpu.upload(a * s), gpu.upload(b), c)
     mag = np.abs(a).astype(np.float64) @ np.abs(b)
     assert np.all(np.abs(gpu.download(c) / np.float64(s) - a.astype(np.float64) @ b) <= bound(k, mag))
+
+
+@pytest.mark.parametrize("m,n,k", [(512, 10, 256), (100, 32, 200), (65, 17, 129), (64, 33, 128)])
+def test_bias_gradient_of_a_narrow_layer_is_added_in_row_order(gpu, m, n, k):
+    rng = np.random.default_rng(m + n + k)
+    a, b, da, db = operands(G.TN, m, n, k, rng)
+    c, cs = gpu.empty((m, n)), gpu.empty((1, n))
+    gpu.matmul_at_b(gpu.upload(da), gpu.upload(db), c, colsum=cs)
+    mag = np.abs(a).astype(np.float64) @ np.abs(b)
+    assert np.all(np.abs(gpu.download(c) - a.astype(np.float64) @ b) <= bound(k, mag))
+    want = np.add.accumulate(b, axis=0, dtype=np.float32)[-1]  # one by one, left to right: the same bits
+    assert np.array_equal(gpu.download(cs)[0], want)
