@@ -827,16 +827,17 @@ __device__ __forceinline__ void dma_body(const HalfArgs& p) {
   // the remaining MFMAs.  Small tiles are left to the scheduler.
   auto interleave = [&](auto n_vm) {
     constexpr int N_VM = decltype(n_vm)::value;
-    if constexpr (N_DS + N_VM <= N_MF) {
+    constexpr int VG = N_MF >= 32 && N_DS + N_VM > N_MF ? 2 : 1, GROUPS = (N_VM + VG - 1) / VG;  // DMA loads a time
+    if constexpr (N_DS + GROUPS <= N_MF) {
       static_for<0, N_DS>([&](auto) {
         __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // one MFMA
         __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);  // one LDS read
       });
-      static_for<0, N_VM>([&](auto) {
-        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // one MFMA
-        __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);  // one global (DMA) load
+      static_for<0, GROUPS>([&](auto) {
+        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);   // one MFMA
+        __builtin_amdgcn_sched_group_barrier(0x020, VG, 0);  // global (DMA) loads
       });
-      __builtin_amdgcn_sched_group_barrier(0x008, N_MF - N_DS - N_VM, 0);
+      __builtin_amdgcn_sched_group_barrier(0x008, N_MF - N_DS - GROUPS, 0);
     }
   };
 
@@ -977,8 +978,8 @@ __global__ __launch_bounds__(256) void cs_shares_reduce_kernel(const float* __re
 // takes ~2000 cycles to arrive): one 256x256 block or two 128x128 blocks hold
 // that in two stages; where a smaller tile has its CU almost to itself, the
 // deep ring holds four (4000x1000, K 4100 TN on 256 128x128 blocks: 55.5 us in
-// two stages, 45.1 in four).
-constexpr int kDmaBK = 64, kDmaStages = 2, kDeepStages = 4;
+// two stages, 45.1 in four); 256x128 tiles fit three.
+constexpr int kDmaBK = 64, kDmaStages = 2, kDeepStages = 4, kWideStages = 3;
 
 template <int BM, int BN>
 void set_tiles(HalfArgs& a) {
@@ -1046,12 +1047,13 @@ hipError_t launch_regs(hipStream_t s, HalfArgs a, int splits, bool bf16) {
 
 // Tile size (256, 128 or 64) and kernel (direct-to-LDS or register-staged)
 // for a problem: 256x256 blocks when they give at least one block per CU,
-// 128x128 for mid sizes, 64x64 for small ones.  Whole tiles take the
+// 256x128 for one round of them, 128x128 for mid sizes, 64x64 for small ones.
+// Whole tiles take the
 // direct-to-LDS kernel (256x256: two waves per SIMD with 128x64 wave tiles),
 // other sizes its form with bounds; the register-staged kernel is left with
 // rows that are no multiple of 8 halves (the DMA moves 16 aligned bytes).
 struct HalfPath {
-  int tile;
+  int bm, bn;
   bool dma;   // whole tiles
   bool edge;  // direct-to-LDS loads too, but tiles may reach past the edges
   bool deep;  // ... through kDeepStages LDS stages
@@ -1064,23 +1066,41 @@ HalfPath pick_path(const HalfArgs& a, int splits, bool overread_ok) {
   // a whole one (4100x4000, K 1000: 272 blocks 94.5 us, as 1056 128x128
   // blocks 83.8).
   const bool idle_round = (tbig + 255) / 256 * 256 > tbig * 4 / 3;
-  const int tile = tbig >= 256 && !idle_round ? 256 : t128 >= 128 ? 128 : 64;
   // Four stages leave room for one 128x128 block per CU.
-  const bool deep = tile == 64 || (tile == 128 && t128 <= 256);
-  // A ragged N is read past its end only along B's rows (N-contiguous B).
+  const bool deep128 = t128 <= 256;
   const bool addressable = dma_addressable<A_KC, B_KC>(a);
-  const bool dma = full_tiles(a, splits, tile, tile, overread_ok && !B_KC) && addressable;
   // Slices (all but the last) are whole stages, so only the last can be cut by
   // K; every element of a K-contiguous row lies in a whole 8-half chunk.
   const bool short_rows = a.lda <= (1 << 21) && a.ldb <= (1 << 21);  // offsets of a whole tile or stage below 2^31
-  return HalfPath{tile, dma, !dma && addressable && short_rows && a.vec_a && a.vec_b && a.K > 0, deep};
+  const bool edge_ok = addressable && short_rows && a.vec_a && a.vec_b && a.K > 0;
+  auto path = [&](int bm, int bn, bool deep) {
+    // A ragged N is read past its end only along B's rows (N-contiguous B).
+    const bool dma = full_tiles(a, splits, bm, bn, overread_ok && !B_KC) && addressable;
+    return HalfPath{bm, bn, dma, !dma && edge_ok, deep};
+  };
+  if (tbig >= 256 && !idle_round) return path(256, 256, false);
+  // 256x128 blocks (128x64 wave tiles, which read a quarter less LDS per MFMA
+  // than 64x64) where one round of them fills the chip and the epilogue is a
+  // plain store: 2048x2048, K 4096 TN 53.8 us as 256 128x128 blocks, 44.8 this
+  // way; 4096x2048, K 2048 NN 47.7 and 42.5.  With a bias, ReLU or mask to
+  // apply, one block per CU leaves the matrix cores idle meanwhile (the bf16
+  // plan's hidden layers at batch 4096 gained nothing, its dX lost 8%), and NT
+  // at K 1024 lost 4%.
+  if constexpr (!B_KC) {
+    const long long twide = (long long)((a.M + 255) / 256) * ((a.N + 127) / 128) * splits;
+    if ((splits > 1 || a.epi == RT_EPI_NONE) && twide > 192 && twide <= 256) {
+      const HalfPath hp = path(256, 128, false);
+      if (hp.dma || hp.edge) return hp;
+    }
+  }
+  return t128 >= 128 ? path(128, 128, deep128) : path(64, 64, true);
 }
 
 template <bool A_KC, bool B_KC>
 hipError_t launch_half(hipStream_t s, HalfArgs a, int splits, bool bf16, float* cs_scratch, size_t cs_elems,
                        bool overread_ok, bool shares_to_caller) {
   const HalfPath hp = pick_path<A_KC, B_KC>(a, splits, overread_ok);
-  a.n_ragged = hp.dma && a.N % hp.tile != 0;
+  a.n_ragged = hp.dma && a.N % hp.bn != 0;
   if (!hp.dma || splits > 1) a.nf_flag = nullptr;  // gemm_checks_nonfinite says false for these
   // Predicate bits only where the direct epilogue writes or reads them
   // (gemm_relu_bits_ok): never leave them unwritten or ignored silently.
@@ -1089,8 +1109,13 @@ hipError_t launch_half(hipStream_t s, HalfArgs a, int splits, bool bf16, float* 
        (a.relu_bits_out && !(a.epi == RT_EPI_BIAS_RELU && a.out_bf16)) || (a.relu_bits && a.epi != RT_EPI_RELU_MASK)))
     return hipErrorInvalidValue;
   const bool direct = hp.dma || hp.edge;
-  switch (hp.tile) {
+  switch (hp.bm) {
     case 256:
+      if constexpr (!B_KC) {
+        if (hp.bn == 128)  // direct only (pick_path)
+          return launch_dma<256, 128, 2, 2, A_KC, B_KC, kWideStages>(s, a, splits, bf16, hp.edge, cs_scratch, cs_elems,
+                                                                     shares_to_caller);
+      }
       return direct ? launch_dma<256, 256, 2, 4, A_KC, B_KC, kDmaStages>(s, a, splits, bf16, hp.edge, cs_scratch,
                                                                          cs_elems, shares_to_caller)
                     : launch_regs<256, 256, 4, 2, A_KC, B_KC>(s, a, splits, bf16);
@@ -1115,7 +1140,7 @@ int half_share_rows(const HalfArgs& a, int splits, size_t cs_elems, bool have_sc
   if (B_KC || !a.colsum || !have_scratch) return 0;
   const HalfPath hp = pick_path<A_KC, B_KC>(a, splits, overread_ok);
   if (!hp.dma && !hp.edge) return 0;
-  const int tiles_m = (a.M + hp.tile - 1) / hp.tile;
+  const int tiles_m = (a.M + hp.bm - 1) / hp.bm;
   return (tiles_m > 1 && (size_t)splits * tiles_m * a.N <= cs_elems) ? tiles_m : 0;
 }
 
@@ -1183,7 +1208,7 @@ bool gemm_relu_bits_ok(const GemmDesc& d) {
     case RT_NT: hp = pick_path<true, true>(a, 1, d.overread_ok); break;
     default: return false;
   }
-  return hp.dma && a.N % hp.tile == 0;
+  return hp.dma && a.N % hp.bn == 0;
 }
 
 bool gemm_checks_nonfinite(const GemmDesc& d) {

@@ -21,7 +21,7 @@ def rounded(a, dt):
 # K, M and N around the 64-k stage and the 64, 128 and 256 tiles; the last
 # three have odd rows (the register-staged kernel).
 SHAPES = [(8, 8, 8), (65, 72, 56), (66, 64, 72), (129, 136, 200), (1000, 1032, 64), (1500, 2040, 136), (264, 2000, 328),
-          (4100, 4104, 72), (4100, 1000, 520), (63, 65, 67), (130, 1001, 77), (300, 255, 1003)]
+          (4100, 4104, 72), (4100, 1000, 520), (4096, 2048, 192), (4000, 2000, 200), (4096, 2040, 64), (63, 65, 67), (130, 1001, 77), (300, 255, 1003)]
 
 
 @pytest.mark.parametrize("layout", [G.NN, G.TN, G.NT])
