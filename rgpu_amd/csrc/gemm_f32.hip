@@ -1166,12 +1166,14 @@ __global__ __launch_bounds__(T::THREADS, 2) void gemm_f32_opt_upd2_kernel(F32Arg
 
 // The first cs_blocks blocks each take 256 columns of the column sums: they
 // start first, so their chains of loads run under the plane sums; the rest
-// sum the planes (grid-stride over M*N).
+// sum the planes (grid-stride over M*N).  A result that is not finite sets
+// *nf_flag, where one is given: the bf16 plan's overflow check without a pass
+// of its own over the gradients.
 __global__ __launch_bounds__(256) void splitk_reduce_kernel(const float* __restrict__ part, int S, long long stride,
                                                              int M, int N, float* C, int ldc, int epi,
                                                              const float* bias, const float* mask,
                                                              const float* __restrict__ cs_part, int cs_rows,
-                                                             float* cs, int cs_blocks, int vec4) {
+                                                             float* cs, int cs_blocks, int vec4, int* nf_flag) {
   if ((int)blockIdx.x < cs_blocks) {
     const long long j = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     if (j >= N) return;
@@ -1200,6 +1202,7 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(const float* __restr
       }
     }
     cs[j] = v;
+    if (nf_flag != nullptr && !(fabsf(v) <= 3.402823466e38f)) *nf_flag = 1;
     return;
   }
   const int plane_blocks = (int)gridDim.x - cs_blocks;
@@ -1243,6 +1246,7 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(const float* __restr
           if (!(mk[q] > 0.0f)) v[q] = 0.0f;
       }
       *reinterpret_cast<f4*>(C + row * ldc + col) = v;
+      if (nf_flag != nullptr && !finite4(v)) *nf_flag = 1;
     }
     return;
   }
@@ -1278,6 +1282,7 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(const float* __restr
       }
     }
     C[o] = v;
+    if (nf_flag != nullptr && !(fabsf(v) <= 3.402823466e38f)) *nf_flag = 1;
   }
 }
 
@@ -1671,7 +1676,8 @@ hipError_t gemm_pair_launch(hipStream_t s, const GemmDesc& d0, const GemmDesc& d
 
 hipError_t splitk_reduce_launch(hipStream_t s, const float* partials, int splits, long long stride, int M, int N,
                                 void* C, int out_dtype, int ldc, int epi, const float* bias, const void* mask,
-                                int mask_dtype, const float* colsum_partials, float* colsum, int cs_rows) {
+                                int mask_dtype, const float* colsum_partials, float* colsum, int cs_rows,
+                                int* nf_flag) {
   if (out_dtype != RT_F32 || mask_dtype != RT_F32) return hipErrorInvalidValue;
   const long long total = (long long)M * N;
   auto al16 = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
@@ -1683,7 +1689,7 @@ hipError_t splitk_reduce_launch(hipStream_t s, const float* partials, int splits
   const int cs_blocks = colsum != nullptr ? (N + 255) / 256 : 0;
   rt::launch(splitk_reduce_kernel, dim3(blocks + cs_blocks), dim3(256), 0, s, partials, splits, stride, M, N,
              static_cast<float*>(C), ldc, epi, bias, static_cast<const float*>(mask), colsum_partials, cs_rows, colsum,
-             cs_blocks, vec4 ? 1 : 0);
+             cs_blocks, vec4 ? 1 : 0, nf_flag);
   return hipGetLastError();
 }
 

@@ -188,14 +188,14 @@ static void layer_shares(const Layer& Ly, GemmDesc& d) {
 }
 
 static int finish_split(rt_mlp* p, const GemmDesc& d, const char* lbl_red, void* C, int out_dtype, int epi,
-                        const float* bias, const void* mask, int mask_dtype, float* colsum) {
+                        const float* bias, const void* mask, int mask_dtype, float* colsum, int* nf_flag = nullptr) {
   if (d.splits <= 1) return RT_OK;
   rt_ctx* c = p->ctx;
   const int cs_rows = gemm_cs_share_rows(d);
   Launch Lz(c, lbl_red);
   hipError_t e = splitk_reduce_launch(c->stream, p->partials, d.splits, d.split_stride, d.M, d.N, C, out_dtype, d.N,
                                       epi, bias, mask, mask_dtype, cs_rows ? d.cs_scratch : d.colsum_partials,
-                                      colsum, cs_rows);
+                                      colsum, cs_rows, nf_flag);
   if (e != hipSuccess) return hip_fail(c, e, lbl_red);
   return RT_OK;
 }
@@ -651,7 +651,7 @@ int rt_mlp_create(rt_ctx* c, int n_layers, const size_t* dims, const float* cons
   n += opt_launches(p);  // optimizer
   if (p->mixed) {
     n += 1;  // step prologue
-    int unchecked = 0;  // tensors of the layers whose dW GEMM cannot flag non-finite values itself
+    int unchecked = 0;  // tensors of the layers whose dW GEMM (or its reduction) cannot flag non-finite values itself
     int jobs = 0;       // whole dW launches whose db shares the check launch adds
     for (int l = 0; l < n_layers; ++l) {
       const Layer& Ly = p->L[l];
@@ -661,7 +661,7 @@ int rt_mlp_create(rt_ctx* c, int n_layers, const size_t* dims, const float* cons
       layer_shares(Ly, dw);
       dw.nf_flag = p->state + 1;
       const bool job = Ly.splits_dw <= 1 && gemm_cs_share_rows(dw) > 0;
-      if (!gemm_checks_nonfinite(dw)) unchecked += job ? 1 : 2;  // a share job checks its db itself
+      if (Ly.splits_dw <= 1 && !gemm_checks_nonfinite(dw)) unchecked += job ? 1 : 2;  // a share job checks its db itself
       jobs += job;
     }
     // Separate checks, 24 tensors and 32 share jobs per launch.
@@ -750,13 +750,15 @@ int rt_mlp_step(rt_mlp* p, const rt_buf* x, const rt_buf* labels) {
                             (int)Ly.din, ld_dl, RT_EPI_NONE, nullptr, nullptr, RT_F32, p->grad + Ly.b_off,
                             Ly.splits_dw, Ly.dw_parts);
     if (p->mixed) {
-      // The overflow flag is set by the GEMM's own epilogue where it can;
-      // the other layers' dW/db go to the separate check below, which also
-      // adds a whole launch's db shares into db.
+      // The overflow flag is set by the GEMM's own epilogue where it can, and
+      // by the reduction of a split one; the other layers' dW/db go to the
+      // separate check below, which also adds a whole launch's db shares into
+      // db.
       layer_shares(Ly, dw);
       dw.nf_flag = overflow;
-      unchecked[l] = !gemm_checks_nonfinite(dw);
-      if (unchecked[l]) dw.nf_flag = nullptr;
+      const bool checks = gemm_checks_nonfinite(dw);
+      unchecked[l] = !checks && dw.splits <= 1;
+      if (!checks) dw.nf_flag = nullptr;
       const int rows = dw.splits <= 1 ? gemm_cs_share_rows(dw) : 0;
       if (rows > 0) jobs.push_back(ShareJob{Ly.cs_shares, p->grad + Ly.b_off, rows, (int)Ly.dout});
       job[l] = rows > 0;
@@ -822,7 +824,7 @@ int rt_mlp_step(rt_mlp* p, const rt_buf* x, const rt_buf* labels) {
     }
     if (Ly.dw_parts == nullptr) {  // otherwise the optimizer sums the planes
       rc = finish_split(p, dw, Ly.lbl_dw_red.c_str(), p->grad + Ly.w_off, RT_F32, RT_EPI_NONE, nullptr, nullptr,
-                        RT_F32, p->grad + Ly.b_off);
+                        RT_F32, p->grad + Ly.b_off, p->mixed ? overflow : nullptr);
       if (rc) return rc;
     }
   }

@@ -226,11 +226,12 @@ hipError_t gemm_pair_launch(hipStream_t s, const GemmDesc& d0, const GemmDesc& d
 // With cs_rows > 0 colsum_partials holds a split half GEMM's column-sum
 // shares [splits, cs_rows, N] instead: each slice's rows are added in order
 // from zero, then the slices in order (the bits of the GEMM's own shares
-// launch followed by the plain reduction).
+// launch followed by the plain reduction).  A result or column sum that is not
+// finite sets *nf_flag to 1 (nullptr: not checked).
 hipError_t splitk_reduce_launch(hipStream_t s, const float* partials, int splits, long long stride, int M,
                                 int N, void* C, int out_dtype, int ldc, int epi, const float* bias,
                                 const void* mask, int mask_dtype, const float* colsum_partials, float* colsum,
-                                int cs_rows = 0);
+                                int cs_rows = 0, int* nf_flag = nullptr);
 
 // ---------------------------------------------------------------- row / column kernels
 hipError_t colsum_launch(hipStream_t s, const void* src, int dtype, int rows, int cols, float* dst,

@@ -87,3 +87,25 @@ def test_slices(gpu, dt, m, n, k, slices):
     tol = ((k + 31) // 32 + slices + 4) * 2.0 ** -23 * (np.abs(a64).T @ np.abs(b64))
     assert np.all(np.abs(gpu.download(dw) - a64.T @ b64) <= tol)
     assert np.all(np.abs(gpu.download(cs)[0] - b64.sum(0)) <= k * 2.0 ** -24 * np.abs(b64).sum(0))
+
+
+@pytest.mark.parametrize("dims", [[128, 256, 128], [72, 200, 101]])
+@pytest.mark.parametrize("bad", [False, True])
+def test_reduction_of_a_split_gradient_flags_what_is_not_finite(gpu, dims, bad):
+    """Batch 1024: every dW of the plan is summed over K slices, and that
+    reduction alone sets the overflow flag (four columns at a time, or one)."""
+    batch = 1024
+    rng = np.random.default_rng(7)
+    params = []
+    for i, o in zip(dims, dims[1:]):
+        params += [rng.standard_normal((i, o)).astype(np.float32) / 16, np.zeros((1, o), np.float32)]
+    x = rng.standard_normal((batch, dims[0])).astype(np.float32)
+    if bad:
+        x[1000, 5] = np.inf  # one row of the last slice (3e38 times weights of 1/16 would stay finite)
+    y = G.upload_labels(gpu, rng.integers(0, dims[-1], batch).astype(np.uint32))
+    mlp = G.GpuMlp.from_params(gpu, params, batch, 1e-3, precision="bf16", loss_scale=1024.0)
+    w0 = mlp.weights()
+    mlp.step(gpu.upload(x, G.BF16), y)
+    assert mlp.overflow() == bad
+    same = all(np.array_equal(a, b) for a, b in zip(w0, mlp.weights()))
+    assert same == bad
