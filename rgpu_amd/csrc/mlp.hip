@@ -487,8 +487,8 @@ int rt_mlp_create(rt_ctx* c, int n_layers, const size_t* dims, const float* cons
     // plan's hidden outputs are bf16, which the reduction does not write).
     // Forward and dX products of at most 64 rows go whole to the skinny f32
     // kernel instead (one launch, its own epilogue).  The bf16 plan counts
-    // its 256x256 tiles (half_slices): a 1000-class head at batch 4096 has
-    // 64 of them.
+    // its 256x128 tiles (half_slices): a 1000-class head at batch 4096 has
+    // 128 of them.
     if (p->mixed) {
       Ly.splits_fwd = last ? half_slices(batch, Ly.dout, Ly.din) : 1;
       Ly.splits_dw = half_slices(Ly.din, Ly.dout, batch);
