@@ -316,22 +316,30 @@ __device__ void F32Tile<A_KC, B_KC, BN_>::run(const F32Args& p, int bid, int spl
 // products, each exact in the MFMA's f32 accumulator; the three smallest (mid
 // lo, lo mid, lo lo: below 2^-26 of the product, against the 2^-24 that each
 // f32 sum rounds by) are left out, and six v_mfma_f32_16x16x32_bf16 replace
-// eight v_mfma_f32_16x16x4_f32 at 16 times their rate.  The bf16 MFMA keeps
-// subnormals, so the split holds down to |x| ~ 2^-109.
+// eight v_mfma_f32_16x16x4_f32 at 16 times their rate.
+//
+// Operands are split after a multiplication by 2^16: the smallest bit of an
+// f32, 2^-149, is then 2^-133, that of a bf16, so the split is exact down to
+// the last subnormal (the conversions, the remainders and the MFMA keep
+// subnormals); unscaled, an operand below 2^-109 lost its last part and one
+// below 2^-134 was taken as zero.  The sums are scaled back at the end.  What
+// the scale costs at the other end is left to the f32 MFMA: operands of 2^111
+// and sums of 2^96 (8e28) or more become infinities here.
 //
 // Block: 256 threads, 4 waves stacked along M, each 16 TM rows by all BN =
 // 16 TN columns.  A wave loads its own A rows straight into registers in
 // fragment order (nothing shares them) and splits them there; B, which all
 // four waves read, is loaded by the block, split once and put into LDS as
-// three bf16 planes [col][32 k] (16-byte granule j of column c at j ^ ((c >>
-// 2) & 3): conflict-free reads and writes).  Global loads run two K stages of
-// 32 ahead, the split one stage ahead, one barrier per stage.  MFMAs take the
-// operands swapped, so lane (g, r) ends with C(row 16t + r, columns 16u + 4g
-// .. + 3): float4 stores.
+// three bf16 planes [col][64 k] (16-byte granule j of column c at j ^ ((c >>
+// 1) & 7): conflict-free reads and writes).  Stages are 64 k: the global loads
+// of a stage go out one stage ahead, its split runs between the MFMAs of the
+// stage before it, one barrier per stage.  MFMAs take the operands swapped, so
+// lane (g, r) ends with C(row 16t + r, columns 16u + 4g .. + 3): float4 stores.
 //
 // A result that is not finite (an operand was not, or a sum overflowed) says
 // nothing about which: inf - inf in the split, or inf times a zero part.  A
 // wave that sees one computes its tile again with the f32 MFMA.
+constexpr float kSplitScale = 65536.0f, kUnsplit = 1.0f / kSplitScale;
 typedef __bf16 b2 __attribute__((ext_vector_type(2)));
 typedef __bf16 b8 __attribute__((ext_vector_type(8)));
 typedef unsigned int u4 __attribute__((ext_vector_type(4)));
@@ -348,15 +356,22 @@ struct SplitSel {
   }
 };
 
-// Eight f32 values into their three bf16 planes, 7 VALU instructions a pair,
-// in 14 steps of two: step Q of the eight values x (overwritten by their
-// remainders).  Breadth first, so that no step needs the result of the one
-// before it.
-constexpr int kSplitSteps = 14;
+// Eight f32 values times kSplitScale into their three bf16 planes, 9 VALU
+// instructions a pair, in 18 steps of two: step Q of the eight values x
+// (overwritten by their remainders).  Breadth first, so that no step needs the
+// result of the one before it.
+constexpr int kScaleSteps = 4, kSplitSteps = kScaleSteps + 14;
+// The plane that step Q completes, -1 if none.
+constexpr int plane_done(int Q) {
+  return Q == kScaleSteps + 1 ? 0 : Q == kScaleSteps + 7 ? 1 : Q == kScaleSteps + 13 ? 2 : -1;
+}
 template <int Q>
 __device__ __forceinline__ void split_step(float (&x)[8], const SplitSel& sel, u4 (&out)[3]) {
-  constexpr int plane = Q < 6 ? 0 : Q < 12 ? 1 : 2, q = Q % 6;
-  if constexpr (q < 2) {
+  constexpr int s = Q - kScaleSteps, plane = s < 6 ? 0 : s < 12 ? 1 : 2, q = s % 6;
+  if constexpr (s < 0) {
+    x[2 * Q] *= kSplitScale;
+    x[2 * Q + 1] *= kSplitScale;
+  } else if constexpr (q < 2) {
 #pragma unroll
     for (int i = 2 * q; i < 2 * q + 2; ++i)
       out[plane][i] = __builtin_bit_cast(unsigned, __builtin_convertvector((f2{x[2 * i], x[2 * i + 1]}), b2));
@@ -613,8 +628,8 @@ __device__ void F32Split<TM, TN, A_KC, B_KC>::run(const F32Args& p, int bid, int
       for (int j = 0; j < 8; ++j) cs[i] += fb[i][j];
     }
     split_step<q>(fb[i], sel, bq);
-    if constexpr (q == 1 || q == 7 || q == 13) {  // a plane is complete
-      constexpr int pl = q / 6;
+    constexpr int pl = plane_done(q);
+    if constexpr (pl >= 0) {
       *reinterpret_cast<u4*>(&lds[(buf * 3 + pl) * PLANE + lb[i]]) = bq[pl];
     }
   };
@@ -728,7 +743,7 @@ __device__ void F32Split<TM, TN, A_KC, B_KC>::run(const F32Args& p, int bid, int
   for (int t = 0; t < TM; ++t)
 #pragma unroll
     for (int u = 0; u < TN; ++u) {
-      acc[t][u] += small[t][u];
+      acc[t][u] = (acc[t][u] + small[t][u]) * (kUnsplit * kUnsplit);
       fine = fine && finite4(acc[t][u]);
     }
   if (__any(!fine)) plain_f32(p, acc, row0, n0, kb, ke, g, r);

@@ -137,6 +137,25 @@ def test_small_magnitudes_keep_their_precision(gpu):
     assert np.all(np.abs(gpu.download(c) / np.float64(s) - a.astype(np.float64) @ b) <= bound(k, mag))
 
 
+@pytest.mark.parametrize("layout", [G.NN, G.TN, G.NT])
+@pytest.mark.parametrize("ea,eb", [(-108, 100), (-115, 100), (-128, 100), (-140, 100), (100, -128), (-126, 60),
+                                   (112, -100), (100, 20), (60, 60)])
+def test_magnitudes_at_the_ends_of_the_range(gpu, layout, ea, eb):
+    """Operands whose last bits lie below the smallest bf16, f32 subnormals
+    among them, against large ones, so that the results are ordinary numbers;
+    and operands and sums near the largest f32: the error stays that of a
+    product of ordinary values (an operand's own bits are exact)."""
+    m, n, k = 129, 65, 200
+    rng = np.random.default_rng(ea + 1000)
+    a, b, _, _ = operands(layout, m, n, k, rng)
+    a, b = np.ldexp(a, ea).astype(np.float32), np.ldexp(b, eb).astype(np.float32)
+    c = gpu.empty((m, n))
+    gpu.gemm(layout, gpu.upload(np.ascontiguousarray(a.T if layout == G.TN else a)),
+             gpu.upload(np.ascontiguousarray(b.T if layout == G.NT else b)), c)
+    a64, b64 = a.astype(np.float64), b.astype(np.float64)
+    assert np.all(np.abs(gpu.download(c) - a64 @ b64) <= bound(k, np.abs(a64) @ np.abs(b64)))
+
+
 @pytest.mark.parametrize("m,n,k", [(512, 10, 256), (100, 32, 200), (65, 17, 129), (64, 33, 128)])
 def test_bias_gradient_of_a_narrow_layer_is_added_in_row_order(gpu, m, n, k):
     rng = np.random.default_rng(m + n + k)
