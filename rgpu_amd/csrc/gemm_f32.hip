@@ -336,9 +336,14 @@ __device__ void F32Tile<A_KC, B_KC, BN_>::run(const F32Args& p, int bid, int spl
 // stage before it, one barrier per stage.  MFMAs take the operands swapped, so
 // lane (g, r) ends with C(row 16t + r, columns 16u + 4g .. + 3): float4 stores.
 //
-// A result that is not finite (an operand was not, or a sum overflowed) says
-// nothing about which: inf - inf in the split, or inf times a zero part.  A
-// wave that sees one computes its tile again with the f32 MFMA.
+// An operand that is not finite has hi = itself, so the hi hi products alone
+// give what f32 arithmetic gives (the small ones hold inf - inf and inf times a
+// zero part, and are left out).  A sum or an operand that left the scaled range
+// looks the same: a block that finds a result that is not finite reads its
+// operands once more, and unless their size rules that out its waves compute
+// their tiles again with the f32 MFMA.  2048^3 NN, 98 us: with an infinity or a
+// NaN 187 us, all of a row 209 (recomputed 345 and 490, on the f32 MFMA alone
+// 125), with sums beyond 2^96 377; looking costs 0.1 us where nothing is found.
 constexpr float kSplitScale = 65536.0f, kUnsplit = 1.0f / kSplitScale;
 typedef __bf16 b2 __attribute__((ext_vector_type(2)));
 typedef __bf16 b8 __attribute__((ext_vector_type(8)));
@@ -401,6 +406,7 @@ struct F32Split {
 
   template <class Epi = NoEpi>
   __device__ static void run(const F32Args& p, int bid, int split, float* smem, const Epi& e = Epi{});
+  __device__ static bool may_overflow(const F32Args& p, int m0, int n0, int kb, int ke, float* smem);
   __device__ static void plain_f32(const F32Args& p, f4 (&acc)[TM][TN], int row0, int n0, int kb, int ke, int g,
                                    int r);
   // The k that element e of granule j stands for within a stage.  An MFMA may
@@ -416,8 +422,83 @@ __device__ inline bool finite4(const f4& v) {
          fabsf(v[3]) <= 3.402823466e38f;
 }
 
-// The wave's tile with v_mfma_f32_16x16x4_f32, operands element by element
-// from memory (zero outside): only for tiles that came out non-finite.
+// 16 k of T row (or column) tiles of an operand from k0: lane (g, r) gets rows
+// row0 + 16t + r (past the last one, that one again), k0 + 4g .. + 3; unless
+// WHOLE, zero from ke on.
+template <bool KC, bool WHOLE, int T>
+__device__ __forceinline__ void load_16k(const float* base, int ld, int row0, int rows, int k0, int ke, int g, int r,
+                                         float (&x)[T][4]) {
+  const int k = k0 + 4 * g;
+#pragma unroll
+  for (int t = 0; t < T; ++t) {
+    const int row = min(row0 + 16 * t + r, rows - 1);
+    const float* src = KC ? base + (long long)row * ld + k : base + (long long)k * ld + row;
+    if constexpr (KC && WHOLE) {
+      __builtin_memcpy(x[t], src, 16);
+    } else {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) x[t][j] = WHOLE || k + j < ke ? src[KC ? j : (long long)j * ld] : 0.0f;
+    }
+  }
+}
+
+// The largest finite |x| of R rows (or columns) from row0 of an operand over
+// [kb, ke), the block's share of this thread.
+template <bool KC, int R>
+__device__ __forceinline__ float most_of(const float* base, int ld, int row0, int rows, int kb, int ke) {
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, waves = blockDim.x >> 6, n = ke - kb;
+  float most = 0.0f;
+  auto take = [&](float x) { most = fabsf(x) <= 3.402823466e38f ? fmaxf(most, fabsf(x)) : most; };
+  if constexpr (KC) {
+    for (int i = wave; i < R; i += waves) {
+      const float* src = base + (long long)min(row0 + i, rows - 1) * ld + kb;
+#pragma unroll 4
+      for (int k = 4 * lane; k + 4 <= n; k += 256) {
+        f4 v;
+        __builtin_memcpy(&v, src + k, 16);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) take(v[j]);
+      }
+      if (lane < n % 4) take(src[n - n % 4 + lane]);
+    }
+  } else {
+#pragma unroll
+    for (int i = 0; i < R; i += 64) {
+      const float* src = base + (long long)kb * ld + min(row0 + i + lane % R, rows - 1);
+#pragma unroll 8
+      for (int k = wave; k < n; k += waves) take(src[(long long)k * ld]);
+    }
+  }
+  return most;
+}
+
+// Whether a sum or an operand of the block's tile may have left the range of
+// the scaled products.  If not, a result that is not finite comes from an
+// operand that is not, and is what f32 arithmetic gives.  All threads take part.
+template <int TM, int TN, bool A_KC, bool B_KC>
+__device__ __forceinline__ bool F32Split<TM, TN, A_KC, B_KC>::may_overflow(const F32Args& p, int m0, int n0, int kb,
+                                                                           int ke, float* smem) {
+  float a = most_of<A_KC, BM>(p.A, p.lda, m0, p.M, kb, ke), b = most_of<B_KC, BN>(p.B, p.ldb, n0, p.N, kb, ke);
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) {
+    a = fmaxf(a, __shfl_xor(a, off, 64));
+    b = fmaxf(b, __shfl_xor(b, off, 64));
+  }
+  smem[threadIdx.x] = a;
+  smem[THREADS + threadIdx.x] = b;
+  __syncthreads();
+#pragma unroll
+  for (int w = 0; w < THREADS; w += 64) {
+    a = fmaxf(a, smem[w]);
+    b = fmaxf(b, smem[THREADS + w]);
+  }
+  constexpr float kMost = 1.7014118e38f * kUnsplit;  // 2^127, of a scaled operand
+  return !(a < kMost && b < kMost && (a * kSplitScale) * (b * kSplitScale) * (float)(ke - kb) < 1.7014118e38f);
+}
+
+// The wave's tile with v_mfma_f32_16x16x4_f32, operands straight from memory
+// into registers: only for tiles whose sums may have left the range of the
+// scaled products.  MFMA step j of a chunk takes k = 4g + j in lane group g.
 template <int TM, int TN, bool A_KC, bool B_KC>
 __device__ __forceinline__ void F32Split<TM, TN, A_KC, B_KC>::plain_f32(const F32Args& p, f4 (&acc)[TM][TN], int row0,
                                                                         int n0, int kb, int ke, int g, int r) {
@@ -425,24 +506,22 @@ __device__ __forceinline__ void F32Split<TM, TN, A_KC, B_KC>::plain_f32(const F3
   for (int t = 0; t < TM; ++t)
 #pragma unroll
     for (int u = 0; u < TN; ++u) acc[t][u] = f4{0.0f, 0.0f, 0.0f, 0.0f};
-  for (int k0 = kb; k0 < ke; k0 += 4) {
-    const int k = k0 + g;
-    float a[TM], b[TN];
+  auto chunk = [&](int k0, auto whole) {
+    constexpr bool W = decltype(whole)::value;
+    float a[TM][4], b[TN][4];
+    load_16k<A_KC, W>(p.A, p.lda, row0, p.M, k0, ke, g, r, a);
+    load_16k<B_KC, W>(p.B, p.ldb, n0, p.N, k0, ke, g, r, b);
 #pragma unroll
-    for (int t = 0; t < TM; ++t) {
-      const int m = row0 + 16 * t + r;
-      a[t] = k < ke && m < p.M ? p.A[A_KC ? (long long)m * p.lda + k : (long long)k * p.lda + m] : 0.0f;
-    }
+    for (int j = 0; j < 4; ++j)
 #pragma unroll
-    for (int u = 0; u < TN; ++u) {
-      const int n = n0 + 16 * u + r;
-      b[u] = k < ke && n < p.N ? p.B[B_KC ? (long long)n * p.ldb + k : (long long)k * p.ldb + n] : 0.0f;
-    }
+      for (int t = 0; t < TM; ++t)
 #pragma unroll
-    for (int t = 0; t < TM; ++t)
-#pragma unroll
-      for (int u = 0; u < TN; ++u) acc[t][u] = __builtin_amdgcn_mfma_f32_16x16x4f32(b[u], a[t], acc[t][u], 0, 0, 0);
-  }
+        for (int u = 0; u < TN; ++u)
+          acc[t][u] = __builtin_amdgcn_mfma_f32_16x16x4f32(b[u][j], a[t][j], acc[t][u], 0, 0, 0);
+  };
+  int k0 = kb;
+  for (; k0 + 16 <= ke; k0 += 16) chunk(k0, std::integral_constant<bool, true>{});
+  if (k0 < ke) chunk(k0, std::integral_constant<bool, false>{});
 }
 
 // Stores of a wave tile: lane (g, r) holds rows row0 + 16t + r, columns n0 +
@@ -743,10 +822,21 @@ __device__ void F32Split<TM, TN, A_KC, B_KC>::run(const F32Args& p, int bid, int
   for (int t = 0; t < TM; ++t)
 #pragma unroll
     for (int u = 0; u < TN; ++u) {
-      acc[t][u] = (acc[t][u] + small[t][u]) * (kUnsplit * kUnsplit);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const float x = acc[t][u][e];
+        acc[t][u][e] = (fabsf(x) <= 3.402823466e38f ? x + small[t][u][e] : x) * (kUnsplit * kUnsplit);
+      }
       fine = fine && finite4(acc[t][u]);
     }
-  if (__any(!fine)) plain_f32(p, acc, row0, n0, kb, ke, g, r);
+  // The block's waves look for the cause together: all of them read B.
+  __shared__ int bad[THREADS / 64];
+  const int mine = __any(!fine);
+  if (lane == 0) bad[wave] = mine;
+  __syncthreads();
+  if (__builtin_expect(bad[0] | bad[1] | bad[2] | bad[3], 0)) {
+    if (may_overflow(p, m0, n0, kb, ke, smem) && mine) plain_f32(p, acc, row0, n0, kb, ke, g, r);
+  }
 
   store_tile<TM, TN>(p, acc, row0, n0, g, r, split, e);
 }

@@ -124,6 +124,31 @@ def test_operands_that_are_not_finite(gpu, layout):
     assert np.all(np.abs(np.where(fin, got, 0) - np.where(fin, want, 0)) <= bound(k, mag))
 
 
+@pytest.mark.parametrize("layout", [G.NN, G.TN, G.NT])
+@pytest.mark.parametrize("scale", [0, 50])
+@pytest.mark.parametrize("m,n,k", [(129, 65, 200), (300, 31, 333)])
+def test_infinities_among_finite_operands(gpu, layout, scale, m, n, k):
+    """A tile that holds infinities and NaN takes them from the leading
+    products where its sums cannot overflow (scale 0), and is computed again
+    where they can (2^50: products of 2^100); whole rows of NaN."""
+    rng = np.random.default_rng(m + scale)
+    a, b, _, _ = operands(layout, m, n, k, rng)
+    a, b = np.ldexp(a, scale).astype(np.float32), np.ldexp(b, scale).astype(np.float32)
+    a[3, k - 1], a[17, 5], a[17, 6], a[100, :] = -np.inf, np.inf, np.inf, np.nan
+    b[5, 7], b[6, 7], b[5, 9], b[k - 1, 30] = 1.0, -1.0, 0.0, np.inf  # row 17: inf - inf, inf * 0
+    with np.errstate(all="ignore"):
+        want = a.astype(np.float64) @ b.astype(np.float64)
+        mag = np.abs(np.where(np.isfinite(a), a, 0)).astype(np.float64) @ np.abs(np.where(np.isfinite(b), b, 0))
+    c = gpu.empty((m, n))
+    gpu.gemm(layout, gpu.upload(np.ascontiguousarray(a.T if layout == G.TN else a)),
+             gpu.upload(np.ascontiguousarray(b.T if layout == G.NT else b)), c)
+    got = gpu.download(c)
+    fin = np.isfinite(want)
+    assert np.array_equal(np.isnan(got), np.isnan(want))
+    assert np.array_equal(got[np.isinf(want)], want[np.isinf(want)].astype(np.float32))
+    assert np.all(np.abs(got[fin] - want[fin]) <= bound(k, mag)[fin])
+
+
 def test_small_magnitudes_keep_their_precision(gpu):
     """Operands around 2^-90: the parts of the split stay above the smallest
     subnormal bf16, so the relative error is that of ordinary values."""
