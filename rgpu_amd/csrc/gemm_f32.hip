@@ -666,26 +666,29 @@ __device__ void F32Split<TM, TN, A_KC, B_KC>::run(const F32Args& p, int bid, int
     for (int t = 0; t < TM; ++t)
       load_op(ra, va[t], kk * a_kk, p.lda, std::integral_constant<bool, A_KC>{}, fa[t][kk]);
   };
-  // The remainder's first k is kb: element by element, zero past it.
+  // The remainder's first k is kb: granules inside it whole, the one it ends in
+  // element by element, zero past it.
   auto load_rest = [&]() {
     __amdgpu_buffer_rsrc_t ra, rb;
     rsrcs(kb, ra, rb);
-    auto at = [](const __amdgpu_buffer_rsrc_t& rs, int off, bool in) {
-      return in ? __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rs, off, 0, 0)) : 0.0f;
+    auto granule = [&](const __amdgpu_buffer_rsrc_t& rs, int vo, int ld, auto kc, int j, float (&x)[8]) {
+      if (k_of(j, 7) < rest) return load_op(rs, vo, 0, ld, kc, x);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const int off = vo + 4 * k_of(0, e) * (decltype(kc)::value ? 1 : ld);
+        x[e] = k_of(j, e) < rest ? __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rs, off, 0, 0)) : 0.0f;
+      }
     };
 #pragma unroll
     for (int i = 0; i < UPT; ++i) {
-      const int q = tid + THREADS * i, gr = B_KC ? q % (BK / 8) : q / BN;
-#pragma unroll
-      for (int j = 0; j < 8; ++j) fb[i][j] = at(rb, vb[i] + 4 * k_of(0, j) * (B_KC ? 1 : p.ldb), k_of(gr, j) < rest);
+      const int q = tid + THREADS * i;
+      granule(rb, vb[i], p.ldb, std::integral_constant<bool, B_KC>{}, B_KC ? q % (BK / 8) : q / BN, fb[i]);
     }
 #pragma unroll
     for (int t = 0; t < TM; ++t)
 #pragma unroll
       for (int kk = 0; kk < KK; ++kk)
-#pragma unroll
-        for (int j = 0; j < 8; ++j)
-          fa[t][kk][j] = at(ra, va[t] + kk * a_kk + 4 * k_of(0, j) * (A_KC ? 1 : p.lda), k_of(4 * kk + g, j) < rest);
+        granule(ra, va[t] + kk * a_kk, p.lda, std::integral_constant<bool, A_KC>{}, 4 * kk + g, fa[t][kk]);
   };
 
   // Bias gradient (TN with a colsum target, first M tile): a unit's values are
