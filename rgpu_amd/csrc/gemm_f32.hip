@@ -1437,6 +1437,33 @@ bool row_order_tn(const F32Args& a) {
   return a.splits <= 1 && a.K <= (a.N <= 32 ? 256 : 128) && !dma_better<false, false>(a);
 }
 
+// Products with so short a K that the split tile's prologue (operands split
+// before the first MFMA) costs more than its matrix rate gains, on grids that
+// give every CU a 64x64 block: 640x2033 NN, K 64 7.4 us on the plain f32 tile,
+// 8.6 split, K 96 8.9 and 9.8, K 128 10.4 and 9.8; with twice the blocks up to
+// K 128 (1856x2450 NN 22.8 and 24.1, K 192 30.5 and 28.5), K 192 where both
+// operands lie along K (25.7 and 27.8); K slices of 32 (500x500 in slices of 64
+// 27.4 and 25.3).  Smaller grids take less split at any K (300x200, K 20 4.1
+// and 3.7).  And K of 1 and 2, where the terms the split leaves out are not
+// small against the rounding of the sum: 1.5 and 2.6 units of 2^-24 |A||B| at
+// most, 1.0 and 1.9 here.
+template <bool A_KC, bool B_KC>
+bool short_k(const F32Args& a) {
+  const long long n64 = (a.N + 63) / 64, t64 = (a.M + 63) / 64 * n64 * a.splits;
+  const long long t128 = (a.M + 127) / 128 * n64 * a.splits;
+  const int k = std::min(a.k_per_split, a.K);
+  if (k <= 2) return true;
+  if (t64 < 256 || a.N <= 32) return false;
+  if (a.splits > 1) return k <= 32;
+  return k <= (t128 < 256 ? 96 : A_KC && B_KC ? 192 : 128);
+}
+
+// Products on the plain f32 tile.
+template <bool A_KC, bool B_KC>
+bool plain_tile(const F32Args& a) {
+  return !split_ok(a) || (!A_KC && row_order_tn(a)) || short_k<A_KC, B_KC>(a);
+}
+
 template <class T>
 hipError_t launch_tile(hipStream_t s, F32Args a) {
   a.tiles_m = (a.M + T::BM - 1) / T::BM;
@@ -1572,7 +1599,7 @@ hipError_t dispatch_tile(hipStream_t s, F32Args a) {
   if constexpr (!A_KC) {
     if (row_order_tn(a) && a.N <= 32) return launch_tile<F32Tile<A_KC, B_KC, 32>>(s, a);
   }
-  if (!split_ok(a) || (!A_KC && row_order_tn(a))) return launch_tile<F32Tile<A_KC, B_KC>>(s, a);
+  if (plain_tile<A_KC, B_KC>(a)) return launch_tile<F32Tile<A_KC, B_KC>>(s, a);
   switch (pick_tile(a)) {
     case kT128x64: return launch_tile<F32Split<2, 4, A_KC, B_KC>>(s, a);
     case kT64x64: return launch_tile<F32Split<1, 4, A_KC, B_KC>>(s, a);
@@ -1630,7 +1657,8 @@ hipError_t launch_pair_tn_nt(hipStream_t s, F32Args a0, F32Args a1) {
 template <class F>
 hipError_t by_tn_tile(const F32Args& a, F&& f) {
   if (dma_better<false, false>(a)) return f(F32DmaTile<false, false>{});
-  if (row_order_tn(a)) return a.N <= 32 ? f(F32Tile<false, false, 32>{}) : f(F32Tile<false, false>{});
+  if (row_order_tn(a) && a.N <= 32) return f(F32Tile<false, false, 32>{});
+  if (plain_tile<false, false>(a)) return f(F32Tile<false, false>{});
   switch (pick_tile(a)) {
     case kT128x64: return f(F32Split<2, 4, false, false>{});
     case kT64x64: return f(F32Split<1, 4, false, false>{});
@@ -1773,12 +1801,13 @@ hipError_t gemm_pair_launch(hipStream_t s, const GemmDesc& d0, const GemmDesc& d
     using T0 = decltype(t0);
     if (rank_k_ok(a1)) return launch_pair_tn_nt<T0, F32RankK>(s, a0, a1);
     if (dma_better<true, true>(a1)) return launch_pair_tn_nt<T0, F32DmaTile<true, true>>(s, a0, a1);
+    if (plain_tile<true, true>(a1)) return launch_pair_tn_nt<T0, F32Tile<true, true>>(s, a0, a1);
     return pick_tile(a1) == kT128x64 ? launch_pair_tn_nt<T0, F32Split<2, 4, true, true>>(s, a0, a1)
                                      : launch_pair_tn_nt<T0, F32Split<1, 4, true, true>>(s, a0, a1);
   };
   if (dma_better<false, false>(a0)) return with_dx(F32DmaTile<false, false>{});
-  if (row_order_tn(a0))
-    return a0.N <= 32 ? with_dx(F32Tile<false, false, 32>{}) : with_dx(F32Tile<false, false>{});
+  if (row_order_tn(a0) && a0.N <= 32) return with_dx(F32Tile<false, false, 32>{});
+  if (plain_tile<false, false>(a0)) return with_dx(F32Tile<false, false>{});
   return a0.N <= 32 ? with_dx(F32Split<1, 2, false, false>{}) : with_dx(F32Split<1, 4, false, false>{});
 }
 

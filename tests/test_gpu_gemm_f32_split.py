@@ -49,6 +49,36 @@ def test_product_against_float64(gpu, layout, m, n, k):
         assert np.all(np.abs(gpu.download(cs)[0] - b64.sum(0)) <= (k / 2 + 8) * 2.0 ** -24 * np.abs(b64).sum(0))
 
 
+@pytest.mark.parametrize("layout", [G.NN, G.TN, G.NT])
+@pytest.mark.parametrize("m,n,k", [(257, 133, 1), (257, 33, 2), (640, 2033, 2), (640, 2033, 96), (640, 2033, 97),
+                                   (1856, 1200, 128), (1856, 1200, 129), (1856, 1200, 192), (1856, 1200, 193)])
+def test_short_products_against_float64(gpu, layout, m, n, k):
+    """Both sides of the rule on K.  A product of one k is the rounded product,
+    one of two the rounded sum of a rounded and an exact one, whatever the tile."""
+    rng = np.random.default_rng(m + n + k)
+    a, b, da, db = operands(layout, m, n, k, rng)
+    c = gpu.empty((m, n))
+    gpu.gemm(layout, gpu.upload(da), gpu.upload(db), c)
+    got, a64, b64 = gpu.download(c), a.astype(np.float64), b.astype(np.float64)
+    mag = np.abs(a64) @ np.abs(b64)
+    if k == 1:
+        assert np.array_equal(got, a * b)
+    assert np.all(np.abs(got - a64 @ b64) <= (2.0 * 2.0 ** -24 * mag if k == 2 else bound(k, mag)))
+
+
+@pytest.mark.parametrize("rows,din,dout", [(3000, 900, 40), (2100, 2000, 100), (2100, 2000, 200), (600, 70, 2)])
+def test_pair_of_a_short_product_gives_the_bits_of_its_products(gpu, rows, din, dout):
+    rng = np.random.default_rng(rows)
+    x, d, w = (gpu.upload(rng.standard_normal(s).astype(np.float32)) for s in ((rows, din), (rows, dout), (din, dout)))
+    dx, dw, db = gpu.empty((rows, din)), gpu.empty((din, dout)), gpu.empty((1, dout))
+    gpu.linear_backward(x, d, w, dx, dw, db)
+    dx1, dw1, db1 = gpu.empty((rows, din)), gpu.empty((din, dout)), gpu.empty((1, dout))
+    gpu.matmul_at_b(x, d, dw1, colsum=db1)
+    gpu.matmul_a_bt(d, w, dx1)
+    for got, want in ((dx, dx1), (dw, dw1), (db, db1)):
+        assert gpu.download(got).tobytes() == gpu.download(want).tobytes()
+
+
 @pytest.mark.parametrize("m,n,k", [(129, 65, 200), (256, 128, 576), (300, 77, 1000)])
 def test_epilogues(gpu, m, n, k):
     rng = np.random.default_rng(m + n + k)
