@@ -40,6 +40,15 @@ __device__ inline __amdgpu_buffer_rsrc_t raw_rsrc(const void* base) {
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), (short)0, 0x7fffffff, 0x00020000);
 }
 
+// The byte offset lane_off + uniform_off of a buffer access that may lie past
+// the descriptor's end, on purpose: below 2^32, as the range check sees it, but
+// not below 2^31, so the sum is unsigned.
+__host__ __device__ constexpr int past_end_offset(int lane_off, unsigned uniform_off) {
+  return (int)((unsigned)lane_off + uniform_off);
+}
+// Evaluated by the compiler, which refuses an overflow here.
+static_assert((unsigned)past_end_offset(0x7ffffff0, 0x7ffffff0u) == 0xffffffe0u, "no signed overflow");
+
 // One 16-byte-per-lane DMA from global memory (rsrc + voff + soff bytes) into
 // LDS at lds + 16 * lane.  The scalar offset is made opaque to the optimiser,
 // which would otherwise fold it into a separate VGPR offset per instruction.

@@ -464,13 +464,11 @@ struct DmaOperand {
 #pragma unroll
     for (int i = 0; i < PER_WAVE; ++i) {
       const int par = PAR ? (i & 1) : 0;
-      int vo = voff[par], so = stage_bytes + i * RSTEP * row_bytes;
-      if constexpr (EDGE) {
-        // The whole offset in the vector part: the range check compares that
-        // with the descriptor's size (at most 2^32 - 1, so it cannot wrap).
-        vo = (last ? vlast[par] : vo) + so;
-        so = 0;
-      }
+      int vo = voff[par], so = 0;
+      if constexpr (EDGE)  // all of it in the vector part, which the range check compares with the descriptor's size
+        vo = rt_dev::past_end_offset(last ? vlast[par] : vo, (unsigned)stage_bytes + (unsigned)(i * RSTEP * row_bytes));
+      else
+        so = stage_bytes + i * RSTEP * row_bytes;
       if constexpr (ASM)
         rt_dev::dma16_asm(rsrc, lds + 512 * (i * WAVES + wave), vo, so);
       else
