@@ -1007,13 +1007,20 @@ bool dma_addressable(const HalfArgs& a) {
   return (long long)(A_KC ? a.M : a.K) * a.lda * 2 < lim && (long long)(B_KC ? a.N : a.K) * a.ldb * 2 < lim;
 }
 
+// Whether the M tiles share the column sums of B, each adding some of the K
+// stages, instead of the first adding them all: edge tiles where K is long
+// enough to pay for the launch that adds the shares (1000x1000, K 328 6.6 us
+// unshared, 8.1 shared, K 4100 28.0 and 25.5; 4000x1000, K 1000 21.0 and 19.0;
+// 384x64 in 23 slices of 128 8.8 and 19.5); whole tiles always.
+bool share_colsum(const HalfArgs& a, bool edge) { return !edge || a.k_per_split > 1024; }
+
 template <int BM, int BN, int WGM, int WGN, bool A_KC, bool B_KC, int NS>
 hipError_t launch_dma(hipStream_t s, HalfArgs a, int splits, bool bf16, bool edge, float* cs_scratch = nullptr,
                       size_t cs_scratch_elems = 0, bool shares_to_caller = false) {
   set_tiles<BM, BN>(a);
   // Column sums shared over the M tiles when there are several and room.
   a.cs_parts = nullptr;
-  if (!B_KC && a.colsum && a.tiles_m > 1 && cs_scratch &&
+  if (!B_KC && a.colsum && share_colsum(a, edge) && a.tiles_m > 1 && cs_scratch &&
       (size_t)splits * a.tiles_m * a.N <= cs_scratch_elems)
     a.cs_parts = cs_scratch;
   const dim3 grid(a.tiles_m * a.tiles_n, 1, splits), block(64 * WGM * WGN);
@@ -1137,7 +1144,7 @@ template <bool A_KC, bool B_KC>
 int half_share_rows(const HalfArgs& a, int splits, size_t cs_elems, bool have_scratch, bool overread_ok) {
   if (B_KC || !a.colsum || !have_scratch) return 0;
   const HalfPath hp = pick_path<A_KC, B_KC>(a, splits, overread_ok);
-  if (!hp.dma && !hp.edge) return 0;
+  if ((!hp.dma && !hp.edge) || !share_colsum(a, hp.edge)) return 0;
   const int tiles_m = (a.M + hp.bm - 1) / hp.bm;
   return (tiles_m > 1 && (size_t)splits * tiles_m * a.N <= cs_elems) ? tiles_m : 0;
 }

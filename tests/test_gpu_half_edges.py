@@ -53,6 +53,25 @@ def test_product_bias_mask_and_colsum(gpu, layout, m, n, k, dt):
         assert np.all(np.abs(got - exact * (mask > 0)) <= tol + 2.0 ** -8 * np.abs(exact))
 
 
+@pytest.mark.parametrize("m,n,k", [(200, 72, 1024), (200, 72, 1032), (1000, 264, 1096)])
+@pytest.mark.parametrize("slices", [1, 3])
+def test_column_sums_on_both_sides_of_the_sharing_rule(gpu, m, n, k, slices):
+    """Up to 1024 rows a slice the first M tile adds them, beyond it the M tiles
+    share them: the same sums, to the rounding of their order."""
+    rng = np.random.default_rng(k)
+    a, b = (rounded(rng.standard_normal(s).astype(np.float32), G.BF16) for s in ((k * slices, m), (k * slices, n)))
+    c, cs = gpu.empty((m, n)), gpu.empty((1, n))
+    A, B = gpu.upload(a, G.BF16), gpu.upload(b, G.BF16)
+    if slices == 1:
+        gpu.matmul_at_b(A, B, c, colsum=cs)
+    else:
+        gpu.split_k(A, B, c, gpu.empty((slices * (m * n + n),)), slices, True, colsum=cs)
+    a64, b64 = a.astype(np.float64), b.astype(np.float64)
+    kk = k * slices
+    assert np.all(np.abs(gpu.download(cs)[0] - b64.sum(0)) <= kk * 2.0 ** -24 * np.abs(b64).sum(0))
+    assert np.all(np.abs(gpu.download(c) - a64.T @ b64) <= ((kk + 31) // 32 + 4) * 2.0 ** -23 * (np.abs(a64).T @ np.abs(b64)))
+
+
 @pytest.mark.parametrize("layout", [G.NN, G.TN, G.NT])
 def test_what_lies_past_an_edge_does_not_reach_the_result(gpu, layout):
     """A row of infinities next to another row's K remainder, and operands
