@@ -1068,9 +1068,15 @@ HalfPath pick_path(const HalfArgs& a, int splits, bool overread_ok) {
   const long long tbig = (long long)((a.M + 255) / 256) * ((a.N + 255) / 256) * splits;
   const long long t128 = (long long)((a.M + 127) / 128) * ((a.N + 127) / 128) * splits;
   // A 256x256 block has its CU to itself, so a last round of few blocks costs
-  // a whole one (4100x4000, K 1000: 272 blocks 94.5 us, as 1056 128x128
-  // blocks 83.8).
-  const bool idle_round = (tbig + 255) / 256 * 256 > tbig * 4 / 3;
+  // a whole one.  At most a quarter past the first round 128x128 is faster or
+  // as fast at any K (4608x4096, 288 blocks: K 512 39.5 us and 32.9, K 4096
+  // 174.6 and 168.5; 320 blocks, K 4096 170.3 and 167.2 on one card, 174.8 and
+  // 180.0 on another); beyond that, up to three quarters of the rounds filled,
+  // only over a short K (5632x4096, 352 blocks: K 512 39.9 and 39.1, K 1024
+  // 59.3 and 63.1; 6912x4864, 513 blocks: K 512 65.7 and 62.8, K 1024 95.1 and
+  // 103.5, K 4096 275 and 344).
+  const bool idle_round =
+      (tbig + 255) / 256 * 256 > tbig * 4 / 3 && (a.k_per_split <= 512 || (tbig > 256 && tbig <= 320));
   // Four stages leave room for one 128x128 block per CU.
   const bool deep128 = t128 <= 256;
   const bool addressable = dma_addressable<A_KC, B_KC>(a);

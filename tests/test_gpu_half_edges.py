@@ -53,6 +53,16 @@ def test_product_bias_mask_and_colsum(gpu, layout, m, n, k, dt):
         assert np.all(np.abs(got - exact * (mask > 0)) <= tol + 2.0 ** -8 * np.abs(exact))
 
 
+@pytest.mark.parametrize("m,n,k,dt,layout", [
+    *((4000, 4000, 200, G.BF16, layout) for layout in (G.NN, G.TN, G.NT)),  # 256 blocks with bounds
+    *((4001, 4001, 67, G.BF16, layout) for layout in (G.NN, G.TN, G.NT)),   # register-staged (odd rows)
+    (5112, 4096, 520, G.F16, G.NN), (5632, 4088, 512, G.F16, G.NT),         # 320 and 352 blocks: 128x128 tiles
+    (5632, 4088, 520, G.F16, G.NT)])                                        # 352 blocks over a longer K: 256x256
+def test_large_tiles(gpu, m, n, k, dt, layout):
+    """The 256x256 tiles and the rule for a last round of few of them."""
+    test_product_bias_mask_and_colsum(gpu, layout, m, n, k, dt)
+
+
 @pytest.mark.parametrize("m,n,k", [(200, 72, 1024), (200, 72, 1032), (1000, 264, 1096)])
 @pytest.mark.parametrize("slices", [1, 3])
 def test_column_sums_on_both_sides_of_the_sharing_rule(gpu, m, n, k, slices):
