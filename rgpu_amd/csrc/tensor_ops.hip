@@ -257,7 +257,7 @@ __global__ __launch_bounds__(256) void sum_stage1(const float* __restrict__ x, l
 }
 
 // out[0] = (the parts added) / div: thread t adds parts t, t + 256, ... in
-// order, then a shared-memory tree.  One thread walking the parts alone was a
+// order, then a shared-memory tree over as many threads as there are parts.  One thread walking the parts alone was a
 // chain of dependent loads (512 parts: the whole sum 90 us, 69 us this way).
 __global__ __launch_bounds__(256) void sum_stage2(const float* __restrict__ part, int parts, float div,
                                                   float* __restrict__ out) {
@@ -267,6 +267,7 @@ __global__ __launch_bounds__(256) void sum_stage2(const float* __restrict__ part
   sh[threadIdx.x] = acc;
   __syncthreads();
   for (int w = 128; w > 0; w >>= 1) {
+    if (w >= parts) continue;  // the upper half is zeros
     if ((int)threadIdx.x < w) sh[threadIdx.x] += sh[threadIdx.x + w];
     __syncthreads();
   }
@@ -775,12 +776,15 @@ hipError_t softmax_rows_vjp_launch(hipStream_t s, const float* sm, const float* 
   });
 }
 
-// f(Band or void*) as the loss launch takes it: one block of kLossThreads for
-// a batch of narrow rows that fits it (a second launch, for the parts, costs
-// more: 256 x 10 takes 4.8 us), long or empty rows as null.
+// f(Band or void*) as the loss launch takes it: a thread per row of at most 4
+// columns (256 x 2 takes 3.5 us, 4.6 on kLossThreads),
+// one block of kLossThreads for a batch of narrow rows that fits it (a second
+// launch, for the parts, costs more: 256 x 10 takes 4.8 us), long or empty rows
+// as null.
 template <class F>
 static hipError_t by_loss_shape(long long rows, long long cols, F&& f) {
   if (rows <= 0 || cols <= 0 || cols > kBandCols) return f(static_cast<void*>(nullptr));
+  if (cols <= 4) return f(Band<1, 4, 1, kRowThreads>{});
   if (cols <= 16 && rows <= 256) return f(Band<16, 1, 4, kLossThreads>{});
   return by_row_length(cols, f);
 }
