@@ -521,8 +521,8 @@ __global__ __launch_bounds__(256) void loss_terms_kernel(int kind, const float* 
 // losses.rs:99-115 from the logits in one pass per row: the softmax of
 // softmax_rows_kernel (the same bits), then dir = p − y and the row's loss
 // terms −y·ln(max(p, 1e-12)) (y ≠ 0).  Each thread adds its terms, a block
-// tree adds the threads; with one block the launch also writes value =
-// (0 + total) / div, else each block writes its part for sum_stage2.  dir may
+// tree adds the threads; without `part` (one block) the launch also writes value
+// = (0 + total) / div, else each block writes its part for sum_stage2.  dir may
 // be z.
 template <int T>
 __device__ inline void loss_block_sum(float terms, float* __restrict__ part, float div, float* __restrict__ out) {
@@ -534,7 +534,7 @@ __device__ inline void loss_block_sum(float terms, float* __restrict__ part, flo
     __syncthreads();
   }
   if (threadIdx.x == 0) {
-    if (gridDim.x == 1) out[0] = (0.0f + red[0]) / div;
+    if (part == nullptr) out[0] = (0.0f + red[0]) / div;
     else part[blockIdx.x] = red[0];
   }
 }
@@ -746,33 +746,47 @@ hipError_t scalar_fill_launch(hipStream_t s, const float* scalar, float div, con
   return hipGetLastError();
 }
 
-static dim3 band_grid(long long rows, int per) { return dim3((unsigned)((rows + per - 1) / per)); }
+static long long band_blocks(long long rows, int per) { return (rows + per - 1) / per; }
+
+// f(first row, rows, grid, first block) per launch: a grid holds fewer than
+// 2^32 threads (HIP takes a larger one and runs what is left of its size
+// modulo 2^32), so 2^26 rows of 33 columns and more go in parts.
+template <class F>
+static hipError_t by_grid(long long rows, int per, int threads, F&& f) {
+  const long long most = 0xffffffffLL / threads;
+  for (long long b = 0, n = band_blocks(rows, per); b < n; b += most)
+    f(b * per, std::min(rows - b * per, most * per), dim3((unsigned)std::min(n - b, most)), b);
+  return hipGetLastError();
+}
 
 hipError_t softmax_rows_launch(hipStream_t s, const float* z, float* y, long long rows, long long cols) {
   if (rows <= 0 || cols <= 0) return hipSuccess;
-  if (cols > kBandCols) {
-    rt::launch(softmax_long_rows_kernel, band_grid(rows, kLongRows), dim3(kRowThreads), 0, s, z, y, rows, cols);
-    return hipGetLastError();
-  }
+  if (cols > kBandCols)
+    return by_grid(rows, kLongRows, kRowThreads, [&](long long r0, long long n, dim3 grid, long long) {
+      rt::launch(softmax_long_rows_kernel, grid, dim3(kRowThreads), 0, s, z + r0 * cols, y + r0 * cols, n, cols);
+    });
   return by_row_length(cols, [&](auto band) {
     using B = decltype(band);
-    rt::launch(softmax_rows_kernel<B>, band_grid(rows, B::ROWS), dim3(B::T), 0, s, z, y, rows, (int)cols);
-    return hipGetLastError();
+    return by_grid(rows, B::ROWS, B::T, [&](long long r0, long long n, dim3 grid, long long) {
+      rt::launch(softmax_rows_kernel<B>, grid, dim3(B::T), 0, s, z + r0 * cols, y + r0 * cols, n, (int)cols);
+    });
   });
 }
 
 hipError_t softmax_rows_vjp_launch(hipStream_t s, const float* sm, const float* g, float* dx, long long rows,
                                    long long cols) {
   if (rows <= 0 || cols <= 0) return hipSuccess;
-  if (cols > kBandCols) {
-    rt::launch(softmax_long_rows_vjp_kernel, band_grid(rows, kLongRows), dim3(kRowThreads), 0, s, sm, g, dx, rows,
-               cols);
-    return hipGetLastError();
-  }
+  if (cols > kBandCols)
+    return by_grid(rows, kLongRows, kRowThreads, [&](long long r0, long long n, dim3 grid, long long) {
+      rt::launch(softmax_long_rows_vjp_kernel, grid, dim3(kRowThreads), 0, s, sm + r0 * cols, g + r0 * cols,
+                 dx + r0 * cols, n, cols);
+    });
   return by_row_length(cols, [&](auto band) {
     using B = decltype(band);
-    rt::launch(softmax_rows_vjp_kernel<B>, band_grid(rows, B::ROWS), dim3(B::T), 0, s, sm, g, dx, rows, (int)cols);
-    return hipGetLastError();
+    return by_grid(rows, B::ROWS, B::T, [&](long long r0, long long n, dim3 grid, long long) {
+      rt::launch(softmax_rows_vjp_kernel<B>, grid, dim3(B::T), 0, s, sm + r0 * cols, g + r0 * cols, dx + r0 * cols, n,
+                 (int)cols);
+    });
   });
 }
 
@@ -793,8 +807,8 @@ size_t xent_logits_parts(long long rows, long long cols) {
   size_t n = 1;
   (void)by_loss_shape(rows, cols, [&](auto band) {
     using B = decltype(band);
-    if constexpr (std::is_pointer_v<B>) n = (size_t)std::max<long long>(1, (rows + kLongRows - 1) / kLongRows);
-    else n = band_grid(rows, B::ROWS).x;
+    if constexpr (std::is_pointer_v<B>) n = (size_t)std::max<long long>(1, band_blocks(rows, kLongRows));
+    else n = (size_t)band_blocks(rows, B::ROWS);
     return hipSuccess;
   });
   return n;
@@ -805,16 +819,21 @@ hipError_t xent_logits_launch(hipStream_t s, const float* z, const float* y, flo
                               float dir_scale) {
   const size_t blocks = xent_logits_parts(rows, cols);
   if (blocks > 1 && blocks > scratch_elems) return hipErrorInvalidValue;
-  const dim3 grid((unsigned)blocks);
+  if (blocks > 0x7fffffff) return hipErrorInvalidValue;
+  float* const part = blocks > 1 ? scratch : nullptr;
   hipError_t e = by_loss_shape(rows, cols, [&](auto band) {
     using B = decltype(band);
     if constexpr (std::is_pointer_v<B>)
-      rt::launch(xent_logits_long_kernel, grid, dim3(kRowThreads), 0, s, z, y, dir, rows, cols, scratch, div, out,
-                 dir_scale);
+      // One block where there is nothing to load.
+      return by_grid(std::max(rows, 1LL), kLongRows, kRowThreads, [&](long long r0, long long n, dim3 grid, long long b) {
+        rt::launch(xent_logits_long_kernel, grid, dim3(kRowThreads), 0, s, z + r0 * cols, y + r0 * cols, dir + r0 * cols,
+                   std::min(n, rows), cols, part ? part + b : part, div, out, dir_scale);
+      });
     else
-      rt::launch(xent_logits_kernel<B>, grid, dim3(B::T), 0, s, z, y, dir, rows, (int)cols, scratch, div, out,
-                 dir_scale);
-    return hipGetLastError();
+      return by_grid(rows, B::ROWS, B::T, [&](long long r0, long long n, dim3 grid, long long b) {
+        rt::launch(xent_logits_kernel<B>, grid, dim3(B::T), 0, s, z + r0 * cols, y + r0 * cols, dir + r0 * cols, n,
+                   (int)cols, part ? part + b : part, div, out, dir_scale);
+      });
   });
   if (e == hipSuccess && blocks > 1) {
     rt::launch(sum_stage2, dim3(1), dim3(256), 0, s, scratch, (int)blocks, div, out);

@@ -103,3 +103,30 @@ def test_reduce_to_columns(gpu, rows, cols):
     # added one by one in row order (tensor.rs:399-438): the same bits
     want = np.add.accumulate(np.concatenate([np.zeros((1, cols), np.float32), x]), axis=0, dtype=np.float32)[-1:]
     assert np.array_equal(gpu.download(out).view(np.uint32), want.view(np.uint32))
+
+
+def test_more_rows_than_one_grid_holds(gpu):
+    """2^26 rows of 33 columns need 2^32 threads, the size of a grid: every row
+    of the softmax, its VJP and the loss is computed.
+
+    The sums run over 2.4e9 values, 4096 parts of 256 threads that add 2300
+    each one after another, then a tree: off by at most 2400 * 2^-24 = 1.5e-4 of
+    their terms' magnitude.  The rows past the grid are 6e-2 of them."""
+    rows, cols = 2 ** 26 + 2 ** 22, 33
+    p, one, dx = gpu.zeros((rows, cols)), gpu.zeros((rows, cols)), gpu.empty((rows, cols))
+    total, value = gpu.empty((1,)), gpu.empty((1,))
+    gpu.map("offset", one, one, 1.0)
+    gpu.softmax_rows(p, p)  # of zeros: 1/33 everywhere
+    gpu.sum_all(p, total, rows)
+    assert abs(gpu.download(total)[0] - 1) < 1.5e-4
+    gpu.map("offset", one, dx, 1.0)
+    gpu.softmax_rows_vjp(p, one, dx)  # p (1 - sum p) = 0
+    gpu.map("square", dx, dx)
+    gpu.sum_all(dx, total)
+    assert gpu.download(total)[0] < 1e-3
+    gpu.map("scale", p, one, 0.0)
+    gpu.loss(4, one, p, value, dx)  # logits 0, targets 1/33: ln 33, p - y = 0
+    assert abs(gpu.download(value)[0] / np.log(33) - 1) < 1.5e-4
+    gpu.map("square", dx, dx)
+    gpu.sum_all(dx, total)
+    assert gpu.download(total)[0] < 1e-3
