@@ -111,7 +111,9 @@ def test_more_rows_than_one_grid_holds(gpu):
 
     The sums run over 2.4e9 values, 4096 parts of 256 threads that add 2300
     each one after another, then a tree: off by at most 2400 * 2^-24 = 1.5e-4 of
-    their terms' magnitude.  The rows past the grid are 6e-2 of them."""
+    their terms' magnitude; the loss's last stage, 256 threads that add 70000
+    blocks' parts each, by at most 70300 * 2^-24 = 4.2e-3.  The rows past the
+    grid are 6e-2 of them all."""
     rows, cols = 2 ** 26 + 2 ** 22, 33
     p, one, dx = gpu.zeros((rows, cols)), gpu.zeros((rows, cols)), gpu.empty((rows, cols))
     total, value = gpu.empty((1,)), gpu.empty((1,))
@@ -126,7 +128,7 @@ def test_more_rows_than_one_grid_holds(gpu):
     assert gpu.download(total)[0] < 1e-3
     gpu.map("scale", p, one, 0.0)
     gpu.loss(4, one, p, value, dx)  # logits 0, targets 1/33: ln 33, p - y = 0
-    assert abs(gpu.download(value)[0] / np.log(33) - 1) < 1.5e-4
+    assert abs(gpu.download(value)[0] / np.log(33) - 1) < 4.2e-3
     gpu.map("square", dx, dx)
     gpu.sum_all(dx, total)
     assert gpu.download(total)[0] < 1e-3
