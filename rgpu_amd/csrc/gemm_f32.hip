@@ -1589,8 +1589,23 @@ hipError_t launch_rank_k(hipStream_t s, F32Args a) {
   return hipGetLastError();
 }
 
+// Rows that one launch of any tile takes: a grid holds fewer than 2^32 threads
+// (HIP runs a larger one modulo 2^32), 2^24 blocks of at least 64 rows.
+constexpr int kMostRows = 1 << 29;
+
 template <bool A_KC, bool B_KC>
 hipError_t dispatch_tile(hipStream_t s, F32Args a) {
+  if (a.M > kMostRows) {
+    F32Args rest = a;
+    a.M = kMostRows;
+    if (hipError_t e = dispatch_tile<A_KC, B_KC>(s, a); e != hipSuccess) return e;
+    rest.M -= kMostRows;
+    rest.A += A_KC ? (long long)kMostRows * a.lda : (long long)kMostRows;
+    rest.C += (long long)kMostRows * a.ldc;
+    if (rest.mask != nullptr) rest.mask += (long long)kMostRows * a.ldc;
+    rest.colsum = nullptr;  // the first part's
+    return dispatch_tile<A_KC, B_KC>(s, rest);
+  }
   if constexpr (A_KC) {
     if (skinny_ok<A_KC, B_KC>(a)) return launch_skinny<B_KC>(s, a);
   }
@@ -1705,6 +1720,7 @@ hipError_t launch_gemm_opt(hipStream_t s, F32Args a, const rt_opt::OptBatch& b, 
 
 bool gemm_opt_supported(const GemmDesc& d, const OptTensor* ts, int nt, const OptParams& P) {
   if (d.in_dtype != RT_F32 || d.layout != RT_TN || d.M <= 0 || d.N <= 0 || d.K <= 0) return false;
+  if (d.M > kMostRows) return false;
   return nt > 0 && (split_ok(make_args(d)) || row_order_tn(make_args(d))) && optimizer_fits_cache(ts, nt, P);
 }
 
@@ -1788,6 +1804,7 @@ hipError_t gemm_opt_update2_launch(hipStream_t s, const GemmDesc& d0, const OptT
 bool gemm_pair_supported(const GemmDesc& d0, const GemmDesc& d1) {
   if (d0.in_dtype != RT_F32 || d1.in_dtype != RT_F32) return false;
   if (d0.layout != RT_TN || d1.layout != RT_NT || d1.splits > 1) return false;
+  if (d0.M > kMostRows || d1.M > kMostRows) return false;
   // Where the dW alone does not fill the chip with the largest tile.
   const F32Args a0 = make_args(d0), a1 = make_args(d1);
   return (split_ok(a0) || row_order_tn(a0)) && split_ok(a1) && pick_tile(a0) != kT128x64;

@@ -221,3 +221,18 @@ def test_bias_gradient_of_a_narrow_layer_is_added_in_row_order(gpu, m, n, k):
     assert np.all(np.abs(gpu.download(c) - a.astype(np.float64) @ b) <= bound(k, mag))
     want = np.add.accumulate(b, axis=0, dtype=np.float32)[-1]  # one by one, left to right: the same bits
     assert np.array_equal(gpu.download(cs)[0], want)
+
+
+@pytest.mark.parametrize("layout", [G.NN, G.TN, G.NT])
+def test_more_rows_than_one_grid_holds(gpu, layout):
+    """2^30 rows of one column, the most the entry point takes, need 2^24 blocks
+    of 256 threads: every row is computed.  Sums of ones are exact."""
+    m = 2 ** 30
+    a, c, total = gpu.zeros((1, m) if layout == G.TN else (m, 1)), gpu.zeros((m, 1)), gpu.empty((1,))
+    gpu.map("offset", a, a, 1.0)
+    cs = gpu.empty((1, 1)) if layout == G.TN else None
+    gpu.gemm(layout, a, gpu.upload(np.full((1, 1), 2, np.float32)), c, colsum=cs)
+    gpu.sum_all(c, total, m)
+    assert gpu.download(total)[0] == 2
+    if cs is not None:
+        assert gpu.download(cs)[0, 0] == 2
