@@ -642,6 +642,15 @@ __device__ __forceinline__ void store_edge(const HalfArgs& p, const f4 (&acc)[TM
   const int epi = partial ? RT_EPI_NONE : p.epi;
   const bool vec = p.ldc % 4 == 0 && (reinterpret_cast<uintptr_t>(out_bf16 ? (void*)Ch : (void*)Cf) & 15) == 0;
   const bool vec_mask = p.ldc % 4 == 0 && (reinterpret_cast<uintptr_t>(p.mask) & 15) == 0;
+  // The bias once for all rows, ahead of the stores (a load in front of each
+  // store waited for it: 448x5248, K 64 NT 14.7 us, 22x64, K 64 4.6).
+  f4 bias[TN];
+  if (epi == RT_EPI_BIAS || epi == RT_EPI_BIAS_RELU) {
+#pragma unroll
+    for (int u = 0; u < TN; ++u)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) bias[u][e] = p.bias[min(n0 + 16 * u + 4 * g + e, p.N - 1)];
+  }
   static_for<0, TM>([&](auto tc) {
     constexpr int t = decltype(tc)::value;
     const int row = row0 + 16 * t + r;
@@ -656,7 +665,7 @@ __device__ __forceinline__ void store_edge(const HalfArgs& p, const f4 (&acc)[TM
       if (epi == RT_EPI_BIAS || epi == RT_EPI_BIAS_RELU) {
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-          if (e < nv) v[e] = v[e] + p.bias[col + e];
+          v[e] = v[e] + bias[u][e];
           if (epi == RT_EPI_BIAS_RELU) v[e] = fmaxf(v[e], 0.0f);
         }
       } else if (epi == RT_EPI_RELU_MASK) {
