@@ -790,15 +790,17 @@ hipError_t softmax_rows_vjp_launch(hipStream_t s, const float* sm, const float* 
   });
 }
 
-// f(Band or void*) as the loss launch takes it: a thread per row of at most 4
-// columns (256 x 2 takes 3.5 us, 4.6 on kLossThreads),
-// one block of kLossThreads for a batch of narrow rows that fits it (a second
-// launch, for the parts, costs more: 256 x 10 takes 4.8 us), long or empty rows
-// as null.
+// f(Band or void*) as the loss launch takes it: a thread per row of at most 7
+// columns (256 x 2 3.5 us, 4.6 on kLossThreads; 256 x 5 4.0 and 4.6; 300000 x 5
+// 10.5, 21.6 on lane groups; at 8 columns 18.9 and 22.2, but 256 x 8 5.1 and
+// 4.7), one block of kLossThreads for a batch of narrow rows that fits it (a
+// second launch, for the parts, costs more: 256 x 10 takes 4.8 us, 257 x 10
+// 6.8), long or empty rows as null.
 template <class F>
 static hipError_t by_loss_shape(long long rows, long long cols, F&& f) {
   if (rows <= 0 || cols <= 0 || cols > kBandCols) return f(static_cast<void*>(nullptr));
   if (cols <= 4) return f(Band<1, 4, 1, kRowThreads>{});
+  if (cols <= 7) return f(Band<1, 8, 1, kRowThreads>{});
   if (cols <= 16 && rows <= 256) return f(Band<16, 1, 4, kLossThreads>{});
   return by_row_length(cols, f);
 }

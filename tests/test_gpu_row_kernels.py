@@ -77,6 +77,14 @@ def test_xent_from_logits_blocks(gpu, rows, cols):
     assert abs(value - want) <= 2e-6 * max(1.0, abs(want))
 
 
+@pytest.mark.parametrize("cols", [2, 4, 5, 7, 8])
+@pytest.mark.parametrize("rows", [1, 255, 256, 257])
+def test_xent_from_logits_narrow_rows(gpu, rows, cols):
+    """A thread per row up to 7 columns, lane groups from 8 on, and one block
+    or several."""
+    test_xent_from_logits_blocks(gpu, rows, cols)
+
+
 def test_rows_that_are_not_finite(gpu):
     """A NaN or +inf makes its own row NaN, a row of -inf too; -inf next to
     finite values is a probability of zero.  Other rows are untouched."""
