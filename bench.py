@@ -52,6 +52,7 @@ sys.path.insert(0, ROOT)
 
 PEAK_F32_TFLOPS = 157.3   # MI355X dense f32 matrix
 PEAK_BF16_TFLOPS = 2500.0  # MI355X dense bf16 matrix
+PEAK_F32_SPLIT_TFLOPS = PEAK_BF16_TFLOPS / 6  # an f32 product as six bf16 ones (gemm_f32.hip, F32Split)
 PEAK_HBM_GBS = 8000.0
 REF_GPU_MS_B2048 = 6.89   # rtensor GPU step at batch 2048 (README.md:53), RTX 4070 Laptop
 
@@ -84,6 +85,15 @@ def label_flops(label, dims, batch):
             l = int(label[len(pre):])
             return 2 * batch * dims[l] * dims[l + 1]
     return 0
+
+
+def label_peak(label, dims, batch):
+    """Peak TFLOP/s of the matrix units that a plan launch's f32 products run
+    on: products over more than 512 k are split over the bf16 units, shorter
+    ones (whole 64x64 tiles, as here) stay on the f32 ones."""
+    l = int(label[label.index("_l") + 2:])
+    k = {"fwd": (dims[l],), "dw": (batch,), "dx": (dims[l + 1],), "dwdx": (batch, dims[l + 1])}[label[:label.index("_l")]]
+    return PEAK_F32_SPLIT_TFLOPS if min(k) > 512 else PEAK_F32_TFLOPS
 
 
 def traffic_for(label, section=None, key="bytes_per_launch"):
@@ -716,8 +726,11 @@ def main():
     flops = label_flops(name, DIMS, BATCH)
     if flops:
         achieved = flops / (avg_ms * 1e-3) / 1e12
-        roof = {"kernel": name, "bound": "mfma", "achieved": round(achieved, 2), "peak": PEAK_F32_TFLOPS,
-                "unit": "TFLOP/s", "frac": round(achieved / PEAK_F32_TFLOPS, 4), "traffic": traffic_for(name),
+        peak = label_peak(name, DIMS, BATCH)
+        roof = {"kernel": name, "bound": "mfma", "achieved": round(achieved, 2), "peak": round(peak, 1),
+                "peak_is": "dense bf16 matrix / 6 (an f32 product as six bf16 ones)" if peak != PEAK_F32_TFLOPS
+                else "dense f32 matrix",
+                "unit": "TFLOP/s", "frac": round(achieved / peak, 4), "traffic": traffic_for(name),
                 "traffic_source": "profiles/pmc_traffic.json: rocprofv3 --pmc FETCH_SIZE and WRITE_SIZE of "
                                   "bench.py --only step, scaled by a copy kernel of known size",
                 "flops_per_launch": flops, "avg_us": round(avg_ms * 1e3, 2)}

@@ -35,6 +35,12 @@ def test_step_flops_and_compulsory_bytes():
     assert bench.label_flops("optimizer", d, b) == 0
 
 
+def test_each_launch_is_held_against_the_units_it_runs_on():
+    d, b = bench.DIMS, bench.BATCH
+    assert bench.label_peak("dwdx_l1", d, b) == bench.label_peak("fwd_l1", d, b) == bench.PEAK_BF16_TFLOPS / 6
+    assert bench.label_peak("fwd_l0", d, b) == bench.PEAK_F32_TFLOPS
+
+
 def test_reported_traffic_comes_from_the_committed_counts():
     with open(os.path.join(ROOT, "profiles", "pmc_traffic.json")) as f:
         doc = json.load(f)
