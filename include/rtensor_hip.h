@@ -107,7 +107,9 @@ int rt_convert(rt_ctx* ctx, const rt_buf* src, rt_buf* dst);
  * f32, or bf16 for half inputs.  aux is the bias [1, N] for RT_EPI_BIAS*,
  * or the mask source [M, N] for RT_EPI_RELU_MASK, else NULL.  colsum, if not
  * NULL, receives f32 column sums of B over K (= 1ᵀ·B, the bias gradient when
- * B is δ): supported for RT_TN. */
+ * B is δ): supported for RT_TN.  Products of f32 have f32 accuracy over the
+ * whole range, subnormal operands included, whichever matrix units they run on;
+ * infinities and NaN propagate as in f32 arithmetic. */
 int rt_gemm(rt_ctx* ctx, rt_layout layout, const rt_buf* a, const rt_buf* b, rt_buf* c,
             rt_epilogue epi, const rt_buf* aux, rt_buf* colsum);
 
@@ -325,8 +327,8 @@ int rt_softmax_rows_vjp(rt_ctx* ctx, const rt_buf* s, const rt_buf* g, rt_buf* d
  * skip) = sign(d), p − y, or (c − y)/(c(1 − c)) with c = clamp(p, 1e-7,
  * 1 − 1e-7).  The loss node's VJP is rt_fill_scaled(g, batch, dir).  y is
  * NULL for RT_LOSS_MAE (p is already pred − target).  RT_LOSS_SOFTMAX_XENT_LOGITS
- * takes the logits as p and needs dir; its row sums are added before the
- * tree, so its value may differ from RT_LOSS_SOFTMAX_XENT's in the last bits. */
+ * takes the logits as p and needs dir; its terms are added in a tree of their
+ * own, so its value may differ from RT_LOSS_SOFTMAX_XENT's in the last bits. */
 int rt_loss(rt_ctx* ctx, rt_loss_kind kind, const rt_buf* p, const rt_buf* y, rt_buf* value, rt_buf* dir);
 
 /* Gpu::zeros without the zero fill (contents undefined), for op outputs

@@ -12,7 +12,7 @@
 //   F32Dma      v_mfma_f32_16x16x4_f32 fed by direct-to-LDS loads: whole 64x64
 //               tiles over a short K (dma_better)
 //   F32Tile     the same MFMA, register-staged, any shape: weight gradients
-//               over few rows (row_order_tn)
+//               over few rows (row_order_tn), short products (short_k)
 //   F32RankK    dX of a narrow layer (K <= 16)
 //   gemm_f32_skinny_kernel   at most 64 rows of output
 //
@@ -83,8 +83,8 @@ __device__ inline f4 load4(const float* base, int ld, int row, int col, int rows
 
 // One block's work: tile `bid` (already XCD-renumbered, in [0, tiles)) of
 // K slice `split`, with v_mfma_f32_16x16x4_f32, every access bounds-checked:
-// short weight gradients (row_order_tn) and operands whose rows are too long
-// for the tiles below.
+// short weight gradients (row_order_tn), other short products (short_k) and
+// operands whose rows are too long for the tiles below.
 //
 // Four wave64s in a 2x2 arrangement, K staged through LDS 32 at a time,
 // double-buffered with register staging (one barrier per K step).  A 16x16x4
@@ -296,12 +296,6 @@ __device__ void F32Tile<A_KC, B_KC, BN_>::run(const F32Args& p, int bid, int spl
         }
       }
       float* dst = Cout + (long long)row * p.ldc + col0;
-      if constexpr (TN == 4) {
-        if (p.vec_c && col0 + 3 < p.N) {
-          *reinterpret_cast<f4*>(dst) = f4{v[0], v[1], v[2], v[3]};
-          continue;
-        }
-      }
 #pragma unroll
       for (int u = 0; u < TN; ++u)
         if (col0 + u < p.N) dst[u] = v[u];
@@ -1431,10 +1425,10 @@ bool dma_better(const F32Args& a) {
 // TN products (weight gradients) over at most 128 rows, or 256 where N is at
 // most 32 columns, that dma_better leaves out stay on the plain f32 tile, whose
 // column sums are added row by row: the bias gradient of a small batch then has
-// the bits of the reference's left-to-right sum.  It costs nothing there: a
-// narrow output layer (512x10, K 256) takes 10.1 us on the 64x32 tile (10.6
-// before the split tile, 12.8 on the 64x64 one), a launch of few blocks either
-// way.
+// the bits of the reference's left-to-right sum, as it had before the split
+// tile.  That is what the limits are for; it costs the narrow layer's launch
+// some time near them (512x10: K 128 6.2 us, K 256 9.8, K 257 6.5 on the split
+// tile, 11.5 on this one).
 bool row_order_tn(const F32Args& a) {
   return a.splits <= 1 && a.K <= (a.N <= 32 ? 256 : 128) && !dma_better<false, false>(a);
 }

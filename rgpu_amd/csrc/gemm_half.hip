@@ -709,10 +709,10 @@ __device__ __forceinline__ void store_edge(const HalfArgs& p, const f4 (&acc)[TM
   });
 }
 
-// Two LDS stages of BKD = 64 k (two MFMA k-steps, kk = 0, 1).  With the
-// fragments of (stage k, kk 0) already in registers, stage k runs as
+// A ring of NS (2, 3 or 4) LDS stages of BKD = 64 k (two MFMA k-steps, kk = 0,
+// 1).  With the fragments of (stage k, kk 0) already in registers, stage k runs as
 //   A: read (k, kk 1) fragments       | MFMAs of (k, kk 0)
-//   B: wait for stage k+1, barrier, DMA stage k+2 into stage k's buffer,
+//   B: wait for stage k+1, barrier, DMA stage k+NS into stage k's buffer,
 //      read (k+1, kk 0) fragments     | MFMAs of (k, kk 1)
 // so every LDS read overlaps MFMAs and there is one barrier per 64 k.  The
 // reads and the DMA are interleaved one per MFMA: a single wave per SIMD
@@ -878,9 +878,9 @@ __device__ __forceinline__ void dma_body(const HalfArgs& p) {
 
   if (nk > 0) {
     u4 fa0[TM], fb0[TN], fa1[TM], fb1[TN];
-    // Every B step waits for everything and issues one stage of DMA (past
-    // the last stage it re-fetches stage nk-1 into a buffer nothing reads),
-    // so the bookkeeping is the same in every stage.
+    // Every B step leaves NS - 2 stages of DMA in flight and issues one more
+    // (past the last stage it re-fetches stage nk-1 into a buffer nothing
+    // reads), so the bookkeeping is the same in every stage.
     issue(0, 0);
     static_for<1, NS>([&](auto ic) { issue(min((int)decltype(ic)::value, nk - 1), decltype(ic)::value); });
     wait_vm<(NS - 1) * PER_STAGE>();
