@@ -325,7 +325,8 @@ __device__ void F32Tile<A_KC, B_KC, BN_>::run(const F32Args& p, int bid, int spl
 // fragment order (nothing shares them) and splits them there; B, which all
 // four waves read, is loaded by the block, split once and put into LDS as
 // three bf16 planes [col][64 k] (16-byte granule j of column c at j ^ ((c >>
-// 1) & 7): conflict-free reads and writes).  Stages are 64 k: the global loads
+// 1) & 7), for the fragment reads; 18 to 25% of the LDS cycles are conflicts,
+// of an LDS that is active 5% of the time).  Stages are 64 k: the global loads
 // of a stage go out one stage ahead, its split runs between the MFMAs of the
 // stage before it, one barrier per stage.  MFMAs take the operands swapped, so
 // lane (g, r) ends with C(row 16t + r, columns 16u + 4g .. + 3): float4 stores.
