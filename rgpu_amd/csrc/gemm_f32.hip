@@ -401,7 +401,7 @@ struct F32Split {
 
   template <class Epi = NoEpi>
   __device__ static void run(const F32Args& p, int bid, int split, float* smem, const Epi& e = Epi{});
-  __device__ static bool may_overflow(const F32Args& p, int m0, int n0, int kb, int ke, float* smem);
+  __device__ static bool may_overflow(const F32Args& p, int m0, int n0, int kb, int ke, float* smem, int tid);
   __device__ static void plain_f32(const F32Args& p, f4 (&acc)[TM][TN], int row0, int n0, int kb, int ke, int g,
                                    int r);
   // The k that element e of granule j stands for within a stage.  An MFMA may
@@ -438,10 +438,11 @@ __device__ __forceinline__ void load_16k(const float* base, int ld, int row0, in
 }
 
 // The largest finite |x| of R rows (or columns) from row0 of an operand over
-// [kb, ke), the block's share of this thread.
+// [kb, ke), thread tid's share of the block's (256 threads).
 template <bool KC, int R>
-__device__ __forceinline__ float most_of(const float* base, int ld, int row0, int rows, int kb, int ke) {
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, waves = blockDim.x >> 6, n = ke - kb;
+__device__ __forceinline__ float most_of(const float* base, int ld, int row0, int rows, int kb, int ke, int tid) {
+  constexpr int waves = 4;
+  const int lane = tid & 63, wave = tid >> 6, n = ke - kb;
   float most = 0.0f;
   auto take = [&](float x) { most = fabsf(x) <= 3.402823466e38f ? fmaxf(most, fabsf(x)) : most; };
   if constexpr (KC) {
@@ -472,15 +473,16 @@ __device__ __forceinline__ float most_of(const float* base, int ld, int row0, in
 // operand that is not, and is what f32 arithmetic gives.  All threads take part.
 template <int TM, int TN, bool A_KC, bool B_KC>
 __device__ __forceinline__ bool F32Split<TM, TN, A_KC, B_KC>::may_overflow(const F32Args& p, int m0, int n0, int kb,
-                                                                           int ke, float* smem) {
-  float a = most_of<A_KC, BM>(p.A, p.lda, m0, p.M, kb, ke), b = most_of<B_KC, BN>(p.B, p.ldb, n0, p.N, kb, ke);
+                                                                           int ke, float* smem, int tid) {
+  float a = most_of<A_KC, BM>(p.A, p.lda, m0, p.M, kb, ke, tid);
+  float b = most_of<B_KC, BN>(p.B, p.ldb, n0, p.N, kb, ke, tid);
 #pragma unroll
   for (int off = 32; off > 0; off >>= 1) {
     a = fmaxf(a, __shfl_xor(a, off, 64));
     b = fmaxf(b, __shfl_xor(b, off, 64));
   }
-  smem[threadIdx.x] = a;
-  smem[THREADS + threadIdx.x] = b;
+  smem[tid] = a;
+  smem[THREADS + tid] = b;
   __syncthreads();
 #pragma unroll
   for (int w = 0; w < THREADS; w += 64) {
@@ -829,13 +831,15 @@ __device__ void F32Split<TM, TN, A_KC, B_KC>::run(const F32Args& p, int bid, int
       }
       fine = fine && finite4(acc[t][u]);
     }
-  // The block's waves look for the cause together: all of them read B.
+  // The block's waves look for the cause together: all of them read B.  (The
+  // thread's index from what the epilogue holds anyway: threadIdx.x, kept for
+  // this alone, cost a spill and the 64x64 TN tile its third wave per SIMD.)
   __shared__ int bad[THREADS / 64];
   const int mine = __any(!fine);
   if (lane == 0) bad[wave] = mine;
   __syncthreads();
   if (__builtin_expect(bad[0] | bad[1] | bad[2] | bad[3], 0)) {
-    if (may_overflow(p, m0, n0, kb, ke, smem) && mine) plain_f32(p, acc, row0, n0, kb, ke, g, r);
+    if (may_overflow(p, m0, n0, kb, ke, smem, 64 * wave + 16 * g + r) && mine) plain_f32(p, acc, row0, n0, kb, ke, g, r);
   }
 
   store_tile<false>(p, acc, row0, n0, g, r, split, e);
