@@ -428,8 +428,10 @@ def test_row_counts_past_int32_are_refused(gpu):
 @pytest.mark.parametrize("m,n,k", [(4096, 4096, 256), (4100, 4000, 96)])
 @pytest.mark.parametrize("dt", [G.BF16, G.F16])
 def test_half_gemm_large_tiles(gpu, m, n, k, dt):
-    # Shapes big enough for the 256x256 block configuration, including ragged
-    # edge tiles; against the float64 product of the same rounded operands.
+    # The 256x256 block configuration on whole tiles, and the 128x128 one with
+    # bounds that 272 blocks over a short K go to (256x256 tiles with ragged
+    # edges: test_gpu_half_edges.py); against the float64 product of the same
+    # rounded operands.
     rng = np.random.default_rng(11)
     a = rng.standard_normal((m, k), dtype=np.float32)
     b = rng.standard_normal((k, n), dtype=np.float32)
